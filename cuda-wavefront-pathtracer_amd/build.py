@@ -22,8 +22,10 @@ CLI = os.path.join(PKG, "pt")
 VIEWER = os.path.join(PKG, "viewer")
 
 HOST_SOURCES = ["host/mesh.cpp", "host/camera.cpp", "host/io.cpp", "host/texture.cpp", "host/bvh.cpp", "host/scene_check.cpp", "host/instances.cpp", "host/envmap.cpp", "host/bvhcache.cpp", "host/setup.cpp", "host/serve.cpp", "capi.cpp"]
-HIP_SOURCES = ["device/renderer.hip", "device/common.hip", "device/kernels_v2.hip", "device/kernels_v4.hip", "device/kernels_v8.hip",
-               "device/hploc.hip", "device/collapse.hip", "device/batch.hip", "device/display.hip"]
+HIP_SOURCES = ["device/renderer.hip", "device/common.hip", "device/hploc.hip", "device/collapse.hip", "device/batch.hip",
+               "device/display.hip"]
+# the traversal kernels, one object per layout and triangle test (the longest compiles start first)
+KERNEL_SOURCES = [("device/kernels_v%d.hip" % v, tri) for v in (8, 4, 2) for tri in (0, 1, 2)]
 CLI_SOURCES = ["app/pt.cpp", "app/viewer.cpp"]
 
 INCLUDES = ["-I" + CSRC, "-I" + os.path.join(ROOT, "include")]
@@ -73,6 +75,11 @@ def build(jobs=8, quiet=False, incremental=False):
     steps = []
     objs = []
     headers = _headers_mtime() if incremental else 0.0
+    for s, tri in KERNEL_SOURCES:
+        o = os.path.join(BUILD, "%s_t%d.o" % (s.replace("/", "_"), tri))
+        if not incremental or _stale(os.path.join(CSRC, s), o, headers):
+            steps.append([hc] + HIP_FLAGS + ["-DCWP_TRI=%d" % tri] + INCLUDES + ["-c", os.path.join(CSRC, s), "-o", o])
+        objs.append(o)
     for s in HOST_SOURCES + CLI_SOURCES:
         o = os.path.join(BUILD, s.replace("/", "_") + ".o")
         if not incremental or _stale(os.path.join(CSRC, s), o, headers):

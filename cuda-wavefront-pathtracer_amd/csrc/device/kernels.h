@@ -1,6 +1,6 @@
 // device/kernels.h - device code of the renderer: constants, path-state and scene records, shading, and the kernel
 // templates per (BVH layout V, triangle test TRI, LDS stack SL). Each layout's kernels are instantiated in exactly one
-// translation unit (kernels_v2.hip, kernels_v4.hip, kernels_v8.hip) through pickKernels<V>; renderer.hip holds the
+// translation unit per triangle test (kernels_v2.hip, kernels_v4.hip, kernels_v8.hip) through pickTri<V, TRI>; renderer.hip holds the
 // layout-independent kernels and the host driver.
 //
 // Design (MI355X-first, not the reference's launch structure):
@@ -281,29 +281,74 @@ __device__ __forceinline__ void enterInstance(const DevScene& S, int k, Vec3 o, 
     if (h.t < before) h.inst = k;
 }
 
-// Two-level traversal over a compressed BVH8 TLAS: the BLAS node step with instances as leaf primitives, each hit
-// leaf's instances entered in slot order; the TLAS's groups share the lane stack with the BLAS traversal above them.
-// The closest hit is the BVH2 TLAS's (both visit every instance whose box the ray enters before the hit).
-template <bool ANY, int TRI, class St>
-__device__ __forceinline__ bool traceInstWide(const DevScene& S, Vec3 o, Vec3 d, float tmin, Hit& h, St& st) {
-    const RayPre r = prepareRay<kTriMT>(o, d, tmin);
-    const int* __restrict__ prim = S.tlasPrim;
-    TravState ts; travBegin(ts, 0);
-    while (!stepBVH8With<ANY>(S.tlas, r, h, st, ts, [&](int k) {
-        enterInstance<8, ANY, TRI>(S, prim[k], o, d, tmin, h, st);
-        return h.tri >= 0;
-    })) {}
-    return h.tri >= 0;
+// the ray of a two-level traversal in the space it is in: the world ray, or the ray in instance `inst`
+template <int TRI>
+__device__ __forceinline__ RayPre instRay(const DevScene& S, int inst, Vec3 o, Vec3 d, float tmin) {
+    if (inst < 0) return prepareRay<TRI>(o, d, tmin);
+    const InstanceRecord* I = S.inst + inst;
+    const Vec4 x[3] = { I->inv[0], I->inv[1], I->inv[2] };
+    return prepareRay<TRI>(xfRowsP(x, o), xfRowsV(x, d), tmin);
 }
 
-// Two-level traversal (reference: travInst, src/accel/traverse_inst.cuh:10-41): the TLAS is a BVH2 whose leaves list
-// instance ids (or, for BVH8 BLASes, a compressed BVH8: traceInstWide); the TLAS's stack entries share the lane stack
-// with the BLAS traversal above them.
+// One node visit of a two-level traversal over a compressed BVH8 TLAS whose leaves name instances. TLAS and BLAS nodes
+// have one form, so a lane in the TLAS and a lane in a BLAS share the node test; only the leaves differ: a BLAS lane
+// tests its triangles, a TLAS lane enters the first instance of its hit leaves (ray to object space, BLAS root next)
+// and leaves the TLAS's group and the other instances on the stack, the latter as an entry marked by its top bit
+// (primitive base, remaining bits). A BLAS whose part of the stack is empty returns to the TLAS. The visiting order
+// per ray is the nested one's (leaves in slot order, each BLAS to its end, then the internal children).
+// What bounds it: the lanes of a wave need different numbers of instances and BLAS nodes (a ray of the 1,001-instance
+// scene enters about 5 instances). With the BLAS traversal nested inside the TLAS step a wave waited for its longest
+// BLAS at every instance: 140.0 ms per 720p frame of 16 samples against 70.3 with the shared step.
+constexpr uint32_t kPendingInst = 0x80000000u;   // groups use the low 16 bits of the high word
+constexpr int kPendingStack = 2;                 // stack entries a TLAS step can add below the BLAS's
+template <bool ANY, int TRI, class St>
+__device__ __forceinline__ bool stepInst8(const DevScene& S, Vec3 o, Vec3 d, float tmin, RayPre& r, Hit& h, St& st,
+                                          TravState& ts) {
+    const Node8 n = testNode8(ts.inst < 0 ? S.tlas : S.nodes, ts.node, r, h.t);
+    uint32_t tm = leafPrims8(n);
+    uint32_t base = (uint32_t)n.triBase;
+    if (ts.inst >= 0)
+        while (tm) {
+            const int j = __builtin_ctz(tm);
+            tm &= tm - 1;
+            if (triTest<TRI>(S.tri, n.triBase + j, r, h)) {
+                h.inst = ts.inst;
+                if (ANY) return true;
+            }
+        }
+    enterGroup8(n, r, st, ts);
+    bool back = false;   // returned to the TLAS in this step: the world ray is made only if a TLAS child is next
+    for (;;) {
+        if (tm) {
+            if (ts.gHits) { st.push(makeGroup(ts.gBase, (ts.gMask << 8) | ts.gHits)); ts.gHits = 0; }
+            const int j = __builtin_ctz(tm);
+            tm &= tm - 1;
+            if (tm) st.push(makeGroup(base, kPendingInst | tm));
+            ts.inst = S.tlasPrim[base + j];
+            st.floor = st.sp;
+            ts.node = S.inst[ts.inst].root;
+            r = instRay<TRI>(S, ts.inst, o, d, tmin);
+            return false;
+        }
+        if (ts.gHits) break;
+        if (st.sp == st.floor) {
+            if (st.sp == 0) return true;
+            ts.inst = -1; st.floor = 0; back = true;
+        }
+        const Group e = st.pop();
+        if ((uint32_t)(e >> 32) & kPendingInst) { tm = (uint32_t)(e >> 32) & ~kPendingInst; base = (uint32_t)e; }
+        else setGroup8(e, ts);
+    }
+    if (back) r = prepareRay<TRI>(o, d, tmin);
+    nextChild8(r, ts);
+    return false;
+}
+
+// Two-level traversal (reference: travInst, src/accel/traverse_inst.cuh:10-41) over a BVH2 TLAS whose leaves list
+// instance ids; the TLAS's stack entries share the lane stack with the BLAS traversal above them.
 template <int V, bool ANY, int TRI, class St>
 __device__ __forceinline__ bool traceInst(const DevScene& S, Vec3 o, Vec3 d, float tmin, Hit& h, St& st) {
     using E = typename StackEntry<V>::type;
-    if constexpr (V == 8)
-        if (S.tlasWide) return traceInstWide<ANY, TRI>(S, o, d, tmin, h, st);
     const RayPre r = prepareRay<kTriMT>(o, d, tmin);
     const float odx = r.o.x * r.ix, ody = r.o.y * r.iy, odz = r.o.z * r.iz;
     int node = S.tlasRoot;
@@ -347,11 +392,20 @@ __device__ __forceinline__ bool traceInst(const DevScene& S, Vec3 o, Vec3 d, flo
     return h.tri >= 0;
 }
 
+// scene forms: one level; two levels with a BVH2 TLAS; two levels with a compressed BVH8 TLAS (and BVH8 BLASes)
+constexpr int kOneLevel = 0, kTlas2 = 1, kTlas8 = 2;
+
 // closest / any hit of one ray in a single- or two-level scene
-template <int V, bool ANY, int TRI, bool INST, class St>
+template <int V, bool ANY, int TRI, int INST, class St>
 __device__ __forceinline__ bool traceRay(const DevScene& S, Vec3 o, Vec3 d, float tmin, Hit& h, St& st) {
     st.sp = 0;
-    if constexpr (INST) return traceInst<V, ANY, TRI>(S, o, d, tmin, h, st);
+    if constexpr (INST == kTlas8) {
+        st.floor = 0;
+        RayPre r = prepareRay<TRI>(o, d, tmin);
+        TravState ts; travBegin(ts, 0);
+        while (!stepInst8<ANY, TRI>(S, o, d, tmin, r, h, st, ts)) {}
+        return h.tri >= 0;
+    } else if constexpr (INST == kTlas2) return traceInst<V, ANY, TRI>(S, o, d, tmin, h, st);
     else return traceScene<V, ANY, TRI>(S, prepareRay<TRI>(o, d, tmin), h, st);
 }
 
@@ -535,31 +589,25 @@ constexpr int kShadeBatch = 32;
 // of buf starting at record regionFirst (queue slot `slot`, the hit so far, the node group and the stack: (slot, t, u,
 // v), (tri, node, group base, group mask), (group hits, stack depth, 0, 0), then two stack entries per Vec4) and mark
 // the hit kHandedOff.
-// One node step of a resumable traversal: the scene's BVH8 (INST false) or, for two-level scenes, the compressed BVH8
-// TLAS, whose leaf primitives are instances entered (each BLAS traversed to the end) within the step; the world ray
-// (o, d, tmin) is needed for the instances. True when the traversal is over.
-template <bool ANY, int TRI, bool INST, class St>
-__device__ __forceinline__ bool resumableStep(const DevScene& S, Vec3 o, Vec3 d, float tmin, const RayPre& r, Hit& h,
+// One node step of a resumable traversal: the scene's BVH8 (INST kOneLevel) or, for two-level scenes, a node of the BVH8
+// TLAS or of the BLAS the ray is in; the world ray (o, d, tmin) is needed to change between them. True when the
+// traversal is over.
+template <bool ANY, int TRI, int INST, class St>
+__device__ __forceinline__ bool resumableStep(const DevScene& S, Vec3 o, Vec3 d, float tmin, RayPre& r, Hit& h,
                                               St& st, TravState& ts) {
-    if constexpr (INST) {
-        const int* prim = S.tlasPrim;
-        return stepBVH8With<ANY>(S.tlas, r, h, st, ts, [&](int k) {
-            enterInstance<8, ANY, TRI>(S, prim[k], o, d, tmin, h, st);
-            return h.tri >= 0;
-        });
-    } else {
-        return stepBVH8<ANY, TRI>(S.nodes, S.tri, r, h, st, ts);
-    }
+    if constexpr (INST) return stepInst8<ANY, TRI>(S, o, d, tmin, r, h, st, ts);
+    else return stepBVH8<ANY, TRI>(S.nodes, S.tri, r, h, st, ts);
 }
-// the ray of a resumable traversal: the world ray for the TLAS (the plain slab test's precomputation) or the BLAS ray
-template <int TRI, bool INST>
-__device__ __forceinline__ RayPre resumableRay(Vec3 o, Vec3 d, float tmin) {
-    return INST ? prepareRay<kTriMT>(o, d, tmin) : prepareRay<TRI>(o, d, tmin);
+// the ray of a resumable traversal in the space it is in
+template <int TRI, int INST>
+__device__ __forceinline__ RayPre resumableRay(const DevScene& S, const TravState& ts, Vec3 o, Vec3 d, float tmin) {
+    if constexpr (INST) return instRay<TRI>(S, ts.inst, o, d, tmin);
+    else return prepareRay<TRI>(o, d, tmin);
 }
 
-template <bool ANY, int TRI, bool INST, class St>
+template <bool ANY, int TRI, int INST, class St>
 __device__ __forceinline__ void stepOrHandOff(const DevScene& S, const DevPaths& P, Vec4* buf, size_t regionFirst,
-                                              int* tailCtr, int slot, Vec3 o, Vec3 d, float tmin, const RayPre& r,
+                                              int* tailCtr, int slot, Vec3 o, Vec3 d, float tmin, RayPre& r,
                                               Hit& h, St& st, TravState& ts) {
     for (;;) {
         if (resumableStep<ANY, TRI, INST>(S, o, d, tmin, r, h, st, ts)) return;
@@ -569,7 +617,9 @@ __device__ __forceinline__ void stepOrHandOff(const DevScene& S, const DevPaths&
     Vec4* rec = buf + first * (size_t)P.tailStride;
     rec[0] = v4(asFloat(slot), h.t, h.u, h.v);
     rec[1] = v4(asFloat(h.tri), asFloat(ts.node), asFloatU(ts.gBase), asFloatU(ts.gMask));
-    rec[2] = v4(asFloatU(ts.gHits), asFloat(st.sp), asFloat(h.inst), 0.f);
+    // two-level scenes: the instance being traversed (25 bits, 0 = the TLAS) and where its stack begins
+    rec[2] = v4(asFloatU(ts.gHits), asFloat(st.sp), asFloat(h.inst),
+                INST ? asFloatU((uint32_t)(ts.inst + 1) | ((uint32_t)st.floor << 25)) : 0.f);
     for (int e = 0; e < st.sp; e += 2) {
         const Group a = st.at(e), b = e + 1 < st.sp ? st.at(e + 1) : (Group)0;
         rec[3 + e / 2] = v4(asFloatU((uint32_t)a), asFloatU((uint32_t)(a >> 32)), asFloatU((uint32_t)b),
@@ -578,22 +628,24 @@ __device__ __forceinline__ void stepOrHandOff(const DevScene& S, const DevPaths&
     h.tri = kHandedOff;
 }
 // The same from the root for a new ray; its records go to region `regionFirst` of buf.
-template <bool ANY, int TRI, bool INST, class St>
+template <bool ANY, int TRI, int INST, class St>
 __device__ __forceinline__ void traceOrHandOff(const DevScene& S, const DevPaths& P, Vec4* buf, size_t regionFirst,
                                                int* tailCtr, int slot, Vec3 o, Vec3 d, float tmin, Hit& h, St& st) {
-    const RayPre r = resumableRay<TRI, INST>(o, d, tmin);
     TravState ts; travBegin(ts, INST ? 0 : S.root);
-    st.sp = 0;
+    RayPre r = prepareRay<TRI>(o, d, tmin);
+    st.sp = 0; st.floor = 0;
     stepOrHandOff<ANY, TRI, INST>(S, P, buf, regionFirst, tailCtr, slot, o, d, tmin, r, h, st, ts);
 }
 
 // A tail record back into a hit, a traversal state and the lane's stack; returns the record's queue slot.
-template <class St>
+template <int INST = kOneLevel, class St>
 __device__ __forceinline__ int resumeRecord(const Vec4* rec, Hit& h, TravState& ts, St& st) {
     const Vec4 a = rec[0], b = rec[1], c = rec[2];
     h.t = a.y; h.u = a.z; h.v = a.w; h.tri = asInt(b.x); h.inst = asInt(c.z);
     ts.node = asInt(b.y); ts.gBase = asUint(b.z); ts.gMask = asUint(b.w); ts.gHits = asUint(c.x);
     const int sp = asInt(c.y);
+    ts.inst = -1; st.floor = 0;
+    if constexpr (INST) { ts.inst = (int)(asUint(c.w) & 0x1FFFFFFu) - 1; st.floor = (int)(asUint(c.w) >> 25); }
     st.sp = 0;
     for (int e = 0; e < sp; e += 2) {
         const Vec4 q = rec[3 + e / 2];
@@ -605,7 +657,7 @@ __device__ __forceinline__ int resumeRecord(const Vec4* rec, Hit& h, TravState& 
 
 // Shading of the traced ray at queue slot `slot` (path i); in the first-bounce sort's depth-0 launch its continuation
 // is staged at its own slot for k_qsort_first instead of being appended.
-template <bool INST, bool FULL>
+template <int INST, bool FULL>
 __device__ __forceinline__ ShadeOut shadeSlot(const DevScene& S, const DevPaths& P, const FrameParams& F, int depth,
                                               int slot, int i, int smpBase, int K, Vec3 o, Vec3 d, const Hit& h) {
     // throughput is fetched after the traversal so that no registers hold it across the traversal loop
@@ -613,9 +665,9 @@ __device__ __forceinline__ ShadeOut shadeSlot(const DevScene& S, const DevPaths&
     ShadeOut res;
     if constexpr (FULL) {
         const float lastPdf = pathLastPdf(P, depth, slot);
-        res = shadeFull<INST>(S, P, F, depth, i, i / K, (uint32_t)(smpBase + i % K), o, d, T, lastPdf, h);
+        res = shadeFull<INST != 0>(S, P, F, depth, i, i / K, (uint32_t)(smpBase + i % K), o, d, T, lastPdf, h);
     } else {
-        res = shadeLegacy<INST>(S, P, F, depth, i, i / K, (uint32_t)(smpBase + i % K), o, d, T, h);
+        res = shadeLegacy<INST != 0>(S, P, F, depth, i, i / K, (uint32_t)(smpBase + i % K), o, d, T, h);
     }
     if (P.firstSort) {   // depth 0: the continuation waits at its own slot for k_qsort_first
         P.qk[slot] = res.cont ? (uint8_t)elevBucket(res.nd) : kNoKey;
@@ -634,11 +686,11 @@ __device__ __forceinline__ ShadeOut shadeSlot(const DevScene& S, const DevPaths&
 // the shadow queue, so a path stays on one XCD (and in its L2) for its whole life. Partition x of the depth-(d+1) queue
 // starts where the depth-d partitions before x end, which bounds it by the rays partition x traced.
 // WAVES: minimum waves per SIMD the register allocation must allow (1 = unconstrained).
-// TAIL (BVH8, single-level scenes): straggler hand-off. After each node visit a wave counts its lanes still tracing;
+// TAIL (BVH8; two-level scenes with a BVH8 TLAS): straggler hand-off. After each node visit a wave counts its lanes still tracing;
 // once fewer than P.tailLanes are, they stop and write their traversal state as tail records (k_bounce_tail resumes
 // them), and the wave shades its finished lanes and takes its next rays. The traversal resumes exactly where it
 // stopped (same hit, node group and stack), so hits and images do not change.
-template <int V, int TRI, int SL, int WAVES, bool INST, bool FULL = false, bool TAIL = false>
+template <int V, int TRI, int SL, int WAVES, int INST, bool FULL = false, bool TAIL = false>
 __global__ void __launch_bounds__(kBlock, WAVES) k_bounce(DevScene S, DevPaths P, const FrameParams* __restrict__ Fp, int depth,
                                                           int smpBase, int K) {
     static_assert(!TAIL || V == 8, "the hand-off resumes BVH8 traversals (two-level scenes: a BVH8 TLAS)");
@@ -709,8 +761,8 @@ __global__ void __launch_bounds__(kFirstTile, WAVES) k_bounce_first(DevScene S, 
             Vec3 o, d; float tmin;
             pathRay(P, F, 0, slot, smpBase, K, i, o, d, tmin);
             Hit h; h.t = 1e30f; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
-            traceRay<V, false, TRI, false>(S, o, d, tmin, h, st);
-            res = shadeSlot<false, FULL>(S, P, F, 0, slot, i, smpBase, K, o, d, h);
+            traceRay<V, false, TRI, kOneLevel>(S, o, d, tmin, h, st);
+            res = shadeSlot<kOneLevel, FULL>(S, P, F, 0, slot, i, smpBase, K, o, d, h);
         }
         const bool cont = res.cont;
         res.cont = false;   // the per-wave appends take the shadow ray and the miss; the tile places the continuation
@@ -728,7 +780,7 @@ __global__ void __launch_bounds__(kFirstTile, WAVES) k_bounce_first(DevScene S, 
 // kernel. LEVEL 1: the traversals its waves handed off, resumed from their records in full waves; with P.tail2 these
 // waves hand their own stragglers on in the same way. LEVEL 2: those, resumed to the end. Each is then shaded and
 // appended like the bounce's own rays.
-template <int TRI, int SL, int WAVES, bool FULL, int LEVEL = 1, bool INST = false>
+template <int TRI, int SL, int WAVES, bool FULL, int LEVEL = 1, int INST = kOneLevel>
 __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_tail(DevScene S, DevPaths P, const FrameParams* __restrict__ Fp,
                                                                int depth, int smpBase, int K) {
     const FrameParams& F = *Fp;
@@ -751,10 +803,10 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_tail(DevScene S, DevPa
         res.cont = false; res.shadow = false; res.miss = false;
         if (k < nt) {
             Hit h; TravState ts;
-            const int slot = resumeRecord(tail + (size_t)k * P.tailStride, h, ts, st);
+            const int slot = resumeRecord<INST>(tail + (size_t)k * P.tailStride, h, ts, st);
             Vec3 o, d; float tmin;
             pathRay(P, F, depth, slot, smpBase, K, i, o, d, tmin);
-            const RayPre r = resumableRay<TRI, INST>(o, d, tmin);
+            RayPre r = resumableRay<TRI, INST>(S, ts, o, d, tmin);
             if (LEVEL == 1 && P.tail2)
                 stepOrHandOff<false, TRI, INST>(S, P, P.tail2, first2, ctr(cnt, part, kCTail2), slot, o, d, tmin, r, h, st, ts);
             else while (!resumableStep<false, TRI, INST>(S, o, d, tmin, r, h, st, ts)) {}
@@ -892,14 +944,14 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_refill(DevScene S, Dev
 
 // Shadow rays of bounce `depth` (partition per XCD as in k_bounce): any hit; unoccluded contributions are added to
 // the path's radiance. The any-hit traversal fits 64 registers without spilling: 8 waves per SIMD.
-// Two-level scenes keep the TLAS ray and the object-space ray live at once: a budget of 6 waves per SIMD (~84
-// registers) is faster than 4 (no spills, less latency hiding) and than 8 (more spills) on the 1,000-instance frame.
+// Two-level scenes keep the world ray beside the ray of the current space: a budget of 6 waves per SIMD (80 registers)
+// beats 5 and 8 (1,001 instances, 720p, 16 samples, BVH8 TLAS: 76.4 ms per frame against 83.6 and 91.7).
 constexpr int kInstWaves = 6;
 // The full integrator's shading (material blend, light choice, BSDF sample) needs about twice the legacy registers;
 // 6 waves per SIMD beat 4 (85 -> 77 ms on a 720p terrain frame) and 8.
 constexpr int kFullWaves = 6;
 
-template <int V, int TRI, int SL, bool INST, bool TAIL = false>
+template <int V, int TRI, int SL, int INST, bool TAIL = false>
 __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow(DevScene S, DevPaths P, int depth) {
     static_assert(!TAIL || V == 8, "the hand-off resumes BVH8 traversals (two-level scenes: a BVH8 TLAS)");
     using E = typename StackEntry<V>::type;
@@ -939,7 +991,7 @@ __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow(DevSce
 
 // The tails of a hand-off shadow kernel: its handed-off any-hit traversals resumed in full waves (LEVEL 1, handing
 // their own stragglers on to tail2 when it is set; LEVEL 2 resumes those to the end).
-template <int TRI, int SL, int LEVEL = 1, bool INST = false>
+template <int TRI, int SL, int LEVEL = 1, int INST = kOneLevel>
 __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow_tail(DevScene S, DevPaths P, int depth) {
     __shared__ Group lds[SL * kBlock];
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
@@ -956,10 +1008,10 @@ __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow_tail(D
         bool vis = false;
         if (k < nt) {
             Hit h; TravState ts;
-            const int pos = resumeRecord(tail + (size_t)k * P.tailStride, h, ts, st);
+            const int pos = resumeRecord<INST>(tail + (size_t)k * P.tailStride, h, ts, st);
             const Vec4 O = P.sO[pos], D = P.sD[pos];
             const Vec3 so = xyz(O), sd = xyz(D);
-            const RayPre r = resumableRay<TRI, INST>(so, sd, 0.f);
+            RayPre r = resumableRay<TRI, INST>(S, ts, so, sd, 0.f);
             if (LEVEL == 1 && P.tail2)
                 stepOrHandOff<true, TRI, INST>(S, P, P.tail2, first2, ctr(cnt, part, kCShadowTail2), pos, so, sd, 0.f, r, h, st, ts);
             else while (!resumableStep<true, TRI, INST>(S, so, sd, 0.f, r, h, st, ts)) {}
@@ -1034,7 +1086,7 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_refill(DevScene S, DevPath
 
 // Closest or any hit of explicit rays (parity and kernel-level entry point); two-level scenes also report the hit
 // instance (-1 on a miss) when hitInst is given.
-template <int V, int TRI, bool ANY, int SL, bool INST>
+template <int V, int TRI, bool ANY, int SL, int INST>
 __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_trace(DevScene S, const Vec4* __restrict__ rays, int n, Vec4* __restrict__ hits,
                                                      int* __restrict__ hitInst, void* spill, int spillCap) {
     using E = typename StackEntry<V>::type;
@@ -1153,10 +1205,10 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_jobs(const DevJobTable
             i = e.i;
             Hit h; h.t = 1e30f; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
             if constexpr (TAIL)
-                traceOrHandOff<false, TRI, false>(J.S, P, P.tail, tailFirst(inStart, part, P.tailLanes), ctr(cnt, part, kCTail),
+                traceOrHandOff<false, TRI, kOneLevel>(J.S, P, P.tail, tailFirst(inStart, part, P.tailLanes), ctr(cnt, part, kCTail),
                                                   slot, o, d, tmin, h, st);
             else
-                traceRay<V, false, TRI, false>(J.S, o, d, tmin, h, st);
+                traceRay<V, false, TRI, kOneLevel>(J.S, o, d, tmin, h, st);
             res = jobShade<FULL>(J, P, depth, slot, e, o, d, h);
         }
         misses += appendResults(P, cnt, part, outStart, depth, i, res);
@@ -1197,8 +1249,8 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_jobs_tail(const DevJob
             const JobEntry e = jobEntry(jobs, base, nJobs, P, depth, slot, o, d, tmin);
             const DevJob& J = jobs[e.j];
             i = e.i;
-            const RayPre r = resumableRay<TRI, false>(o, d, tmin);
-            while (!resumableStep<false, TRI, false>(J.S, o, d, tmin, r, h, st, ts)) {}
+            RayPre r = resumableRay<TRI, kOneLevel>(J.S, ts, o, d, tmin);
+            while (!resumableStep<false, TRI, kOneLevel>(J.S, o, d, tmin, r, h, st, ts)) {}
             res = jobShade<FULL>(J, P, depth, slot, e, o, d, h);
         }
         misses += appendResults(P, cnt, part, outStart, depth, i, res);
@@ -1233,11 +1285,11 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_jobs(const DevJobTable* __
             Hit h; h.t = D.w; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
             bool occluded;
             if constexpr (TAIL) {   // records hold the shadow-queue position as their slot
-                traceOrHandOff<true, TRI, false>(J.S, P, P.tail, tailFirst(start, part, P.tailLanes), ctr(cnt, part, kCShadowTail),
+                traceOrHandOff<true, TRI, kOneLevel>(J.S, P, P.tail, tailFirst(start, part, P.tailLanes), ctr(cnt, part, kCShadowTail),
                                                  start + k, xyz(O), xyz(D), 0.f, h, st);
                 occluded = h.tri != -1;
             } else {
-                occluded = traceRay<V, true, TRI, false>(J.S, xyz(O), xyz(D), 0.f, h, st);
+                occluded = traceRay<V, true, TRI, kOneLevel>(J.S, xyz(O), xyz(D), 0.f, h, st);
             }
             if (!occluded) {
                 vis = true;
@@ -1278,8 +1330,8 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_jobs_tail(const Table* __r
             const int i = asInt(O.w);
             const DevJob& J = jobs[jobOf(base, nJobs, i)];
             const Vec3 so = xyz(O), sd = xyz(D);
-            const RayPre r = resumableRay<TRI, false>(so, sd, 0.f);
-            while (!resumableStep<true, TRI, false>(J.S, so, sd, 0.f, r, h, st, ts)) {}
+            RayPre r = resumableRay<TRI, kOneLevel>(J.S, ts, so, sd, 0.f);
+            while (!resumableStep<true, TRI, kOneLevel>(J.S, so, sd, 0.f, r, h, st, ts)) {}
             if (h.tri == -1) {
                 vis = true;
                 const Vec4 c = P.sC[pos];
@@ -1399,10 +1451,10 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_roll(const DevStepTabl
             i = e.i;
             Hit h; h.t = 1e30f; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
             if constexpr (TAIL)
-                traceOrHandOff<false, TRI, false>(J.S, P, P.tail, tailFirst(outStart, part, P.tailLanes), ctr(blk, part, kCTail),
+                traceOrHandOff<false, TRI, kOneLevel>(J.S, P, P.tail, tailFirst(outStart, part, P.tailLanes), ctr(blk, part, kCTail),
                                                   code, o, d, tmin, h, st);
             else
-                traceRay<V, false, TRI, false>(J.S, o, d, tmin, h, st);
+                traceRay<V, false, TRI, kOneLevel>(J.S, o, d, tmin, h, st);
             res = rollShade<FULL>(J, P, inSet, code, e, o, d, h, depth);
         }
         camMisses += (int)__builtin_popcountll(__ballot(cam && res.miss));
@@ -1447,10 +1499,10 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_roll_tail(const DevSte
             const RollEntry e = rollEntry(T, base, nJobs, P, inSet, code, o, d, tmin);
             const DevJob& J = jobs[e.j];
             i = e.i;
-            const RayPre r = resumableRay<TRI, false>(o, d, tmin);
+            RayPre r = resumableRay<TRI, kOneLevel>(J.S, ts, o, d, tmin);
             if (LEVEL == 1 && P.tail2)
-                stepOrHandOff<false, TRI, false>(J.S, P, P.tail2, first2, ctr(blk, part, kCTail2), code, o, d, tmin, r, h, st, ts);
-            else while (!resumableStep<false, TRI, false>(J.S, o, d, tmin, r, h, st, ts)) {}
+                stepOrHandOff<false, TRI, kOneLevel>(J.S, P, P.tail2, first2, ctr(blk, part, kCTail2), code, o, d, tmin, r, h, st, ts);
+            else while (!resumableStep<false, TRI, kOneLevel>(J.S, o, d, tmin, r, h, st, ts)) {}
             res = rollShade<FULL>(J, P, inSet, code, e, o, d, h, depth);   // nothing if handed on
         }
         camMisses += (int)__builtin_popcountll(__ballot(cam && res.miss));
@@ -1487,11 +1539,11 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_roll(const DevStepTable* _
             Hit h; h.t = D.w; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
             bool occluded;
             if constexpr (TAIL) {
-                traceOrHandOff<true, TRI, false>(J.S, P, P.tail, tailFirst(start, part, P.tailLanes), ctr(blk, part, kCShadowTail),
+                traceOrHandOff<true, TRI, kOneLevel>(J.S, P, P.tail, tailFirst(start, part, P.tailLanes), ctr(blk, part, kCShadowTail),
                                                  start + k, xyz(O), xyz(D), 0.f, h, st);
                 occluded = h.tri != -1;
             } else {
-                occluded = traceRay<V, true, TRI, false>(J.S, xyz(O), xyz(D), 0.f, h, st);
+                occluded = traceRay<V, true, TRI, kOneLevel>(J.S, xyz(O), xyz(D), 0.f, h, st);
             }
             if (!occluded) {
                 vis = true;
@@ -1525,6 +1577,10 @@ struct Kernels {
     BounceFn bounceInst = nullptr;
     ShadowFn shadowInst = nullptr;
     TraceFn traceCInst = nullptr, traceAInst = nullptr;
+    // the same with a BVH8 TLAS (BVH8 BLASes)
+    BounceFn bounceInst8 = nullptr, bounceFullInst8 = nullptr;
+    ShadowFn shadowInst8 = nullptr;
+    TraceFn traceCInst8 = nullptr, traceAInst8 = nullptr;
     // batched jobs
     JobsFn bounceJobs = nullptr, shadowJobs = nullptr;
     // full material integrator (fused bounce kernel; shadow rays use the legacy shadow kernels)
@@ -1535,12 +1591,12 @@ struct Kernels {
     // rolling batches
     RollFn bounceRoll = nullptr, bounceRollFull = nullptr, shadowRoll = nullptr;
     RollFn bounceRollLane = nullptr, bounceRollFullLane = nullptr;   // per-lane compaction
-    // straggler hand-off (BVH8, single-level scenes): the bounce kernels that hand off and their tail kernels
+    // straggler hand-off (BVH8): the bounce kernels that hand off and their tail kernels
     BounceFn bounceHand = nullptr, bounceTail = nullptr, bounceHandFull = nullptr, bounceTailFull = nullptr;
     ShadowFn shadowHand = nullptr, shadowTail = nullptr;
     BounceFn bounceTail2 = nullptr, bounceTail2Full = nullptr;   // second hand-off level
     ShadowFn shadowTail2 = nullptr;
-    // the same for two-level scenes with a BVH8 TLAS (hand-off between TLAS node steps)
+    // the same for two-level scenes with a BVH8 TLAS
     BounceFn bounceHandInst = nullptr, bounceHandFullInst = nullptr, bounceTailInst = nullptr, bounceTailFullInst = nullptr;
     BounceFn bounceTail2Inst = nullptr, bounceTail2FullInst = nullptr;
     ShadowFn shadowHandInst = nullptr, shadowTailInst = nullptr, shadowTail2Inst = nullptr;
@@ -1555,21 +1611,21 @@ struct Kernels {
 
 template <int V, int TRI, int SL>
 void pickSL(int waves, Kernels& k) {
-    k.bounce = waves >= 8 ? k_bounce<V, TRI, SL, 8, false> : (waves >= 6 ? k_bounce<V, TRI, SL, 6, false> : k_bounce<V, TRI, SL, 1, false>);
+    k.bounce = waves >= 8 ? k_bounce<V, TRI, SL, 8, kOneLevel> : (waves >= 6 ? k_bounce<V, TRI, SL, 6, kOneLevel> : k_bounce<V, TRI, SL, 1, kOneLevel>);
     k.tracePaths = k_trace_paths<V, TRI, SL, kRefill>;
     k.tracePlain = k_trace_paths<V, TRI, SL, kWave>;
-    k.shadow = k_shadow<V, TRI, SL, false>;
+    k.shadow = k_shadow<V, TRI, SL, kOneLevel>;
     k.shadowRefill = k_shadow_refill<V, TRI, SL, kRefill>;
-    k.traceC = k_trace<V, TRI, false, SL, false>;
-    k.traceA = k_trace<V, TRI, true, SL, false>;
-    k.bounceInst = k_bounce<V, TRI, SL, kInstWaves, true>;
-    k.shadowInst = k_shadow<V, TRI, SL, true>;
-    k.traceCInst = k_trace<V, TRI, false, SL, true>;
-    k.traceAInst = k_trace<V, TRI, true, SL, true>;
+    k.traceC = k_trace<V, TRI, false, SL, kOneLevel>;
+    k.traceA = k_trace<V, TRI, true, SL, kOneLevel>;
+    k.bounceInst = k_bounce<V, TRI, SL, kInstWaves, kTlas2>;
+    k.shadowInst = k_shadow<V, TRI, SL, kTlas2>;
+    k.traceCInst = k_trace<V, TRI, false, SL, kTlas2>;
+    k.traceAInst = k_trace<V, TRI, true, SL, kTlas2>;
     k.bounceJobs = k_bounce_jobs<V, TRI, SL, 8>;
     k.shadowJobs = k_shadow_jobs<V, TRI, SL>;
-    k.bounceFull = k_bounce<V, TRI, SL, kFullWaves, false, true>;
-    k.bounceFullInst = k_bounce<V, TRI, SL, kFullWaves, true, true>;
+    k.bounceFull = k_bounce<V, TRI, SL, kFullWaves, kOneLevel, true>;
+    k.bounceFullInst = k_bounce<V, TRI, SL, kFullWaves, kTlas2, true>;
     k.bounceRefill = waves >= 8 ? k_bounce_refill<V, TRI, SL, 8, false, kShadeBatch>
                                 : (waves >= 6 ? k_bounce_refill<V, TRI, SL, 6, false, kShadeBatch> : k_bounce_refill<V, TRI, SL, 4, false, kShadeBatch>);
     k.bounceRefillFull = k_bounce_refill<V, TRI, SL, kFullWaves, true, kShadeBatch>;
@@ -1580,24 +1636,29 @@ void pickSL(int waves, Kernels& k) {
     k.bounceRollFullLane = k_bounce_roll<V, TRI, SL, kFullWaves, true, true>;
     k.shadowRoll = k_shadow_roll<V, TRI, SL>;
     if constexpr (V == 8) {
-        k.bounceHand = k_bounce<V, TRI, SL, 8, false, false, true>;
+        k.bounceHand = k_bounce<V, TRI, SL, 8, kOneLevel, false, true>;
         k.bounceTail = k_bounce_tail<TRI, SL, 6, false>;
-        k.bounceHandFull = k_bounce<V, TRI, SL, kFullWaves, false, true, true>;
+        k.bounceHandFull = k_bounce<V, TRI, SL, kFullWaves, kOneLevel, true, true>;
         k.bounceTailFull = k_bounce_tail<TRI, SL, kFullWaves, true>;
-        k.shadowHand = k_shadow<V, TRI, SL, false, true>;
+        k.shadowHand = k_shadow<V, TRI, SL, kOneLevel, true>;
         k.shadowTail = k_shadow_tail<TRI, SL>;
         k.bounceTail2 = k_bounce_tail<TRI, SL, 8, false, 2>;
         k.bounceTail2Full = k_bounce_tail<TRI, SL, kFullWaves, true, 2>;
         k.shadowTail2 = k_shadow_tail<TRI, SL, 2>;
-        k.bounceHandInst = k_bounce<V, TRI, SL, kInstWaves, true, false, true>;
-        k.bounceHandFullInst = k_bounce<V, TRI, SL, kFullWaves, true, true, true>;
-        k.bounceTailInst = k_bounce_tail<TRI, SL, kInstWaves, false, 1, true>;
-        k.bounceTailFullInst = k_bounce_tail<TRI, SL, kFullWaves, true, 1, true>;
-        k.bounceTail2Inst = k_bounce_tail<TRI, SL, kInstWaves, false, 2, true>;
-        k.bounceTail2FullInst = k_bounce_tail<TRI, SL, kFullWaves, true, 2, true>;
-        k.shadowHandInst = k_shadow<V, TRI, SL, true, true>;
-        k.shadowTailInst = k_shadow_tail<TRI, SL, 1, true>;
-        k.shadowTail2Inst = k_shadow_tail<TRI, SL, 2, true>;
+        k.bounceHandInst = k_bounce<V, TRI, SL, kInstWaves, kTlas8, false, true>;
+        k.bounceHandFullInst = k_bounce<V, TRI, SL, kFullWaves, kTlas8, true, true>;
+        k.bounceTailInst = k_bounce_tail<TRI, SL, kInstWaves, false, 1, kTlas8>;
+        k.bounceTailFullInst = k_bounce_tail<TRI, SL, kFullWaves, true, 1, kTlas8>;
+        k.bounceTail2Inst = k_bounce_tail<TRI, SL, kInstWaves, false, 2, kTlas8>;
+        k.bounceTail2FullInst = k_bounce_tail<TRI, SL, kFullWaves, true, 2, kTlas8>;
+        k.bounceInst8 = k_bounce<V, TRI, SL, kInstWaves, kTlas8>;
+        k.bounceFullInst8 = k_bounce<V, TRI, SL, kFullWaves, kTlas8, true>;
+        k.shadowInst8 = k_shadow<V, TRI, SL, kTlas8>;
+        k.traceCInst8 = k_trace<V, TRI, false, SL, kTlas8>;
+        k.traceAInst8 = k_trace<V, TRI, true, SL, kTlas8>;
+        k.shadowHandInst = k_shadow<V, TRI, SL, kTlas8, true>;
+        k.shadowTailInst = k_shadow_tail<TRI, SL, 1, kTlas8>;
+        k.shadowTail2Inst = k_shadow_tail<TRI, SL, 2, kTlas8>;
         k.bounceJobsHand = k_bounce_jobs<V, TRI, SL, 8, false, true>;
         k.bounceJobsHandFull = k_bounce_jobs<V, TRI, SL, kFullWaves, true, true>;
         k.bounceJobsTail = k_bounce_jobs_tail<TRI, SL, 8, false>;
@@ -1628,8 +1689,16 @@ void pickTri(int sl, int waves, Kernels& k) {
     else if (sl == 32) pickSL<V, TRI, 32>(waves, k);
     else pickSL<V, TRI, 16>(waves, k);
 }
-// the kernels of layout V for a triangle test, LDS stack size and bounce register budget (explicitly instantiated once
-// per layout in kernels_v<V>.hip)
+// the kernels of layout V for a triangle test, LDS stack size and bounce register budget (pickTri is instantiated once
+// per layout and triangle test in kernels_v<V>.hip)
+#define CWP_PICK_TRI(V)                                              \
+    extern template void pickTri<V, kTriMT>(int, int, Kernels&);         \
+    extern template void pickTri<V, kTriWoop>(int, int, Kernels&);       \
+    extern template void pickTri<V, kTriWatertight>(int, int, Kernels&);
+CWP_PICK_TRI(2)
+CWP_PICK_TRI(4)
+CWP_PICK_TRI(8)
+#undef CWP_PICK_TRI
 template <int V>
 void pickKernels(int tri, int sl, int waves, Kernels& k) {
     if (tri == kTriMT) pickTri<V, kTriMT>(sl, waves, k);
@@ -1659,9 +1728,6 @@ __global__ void k_step_begin(const DevStepTable* T, int* cnt, int step);
 __global__ void k_reduce_roll(const DevStepTable* __restrict__ T, const Vec4* __restrict__ L);
 __global__ void k_step_end(const int* cnt, int step, unsigned long long* tot);
 
-extern template void pickKernels<2>(int, int, int, Kernels&);
-extern template void pickKernels<4>(int, int, int, Kernels&);
-extern template void pickKernels<8>(int, int, int, Kernels&);
 
 }  // namespace dev
 }  // namespace cwp

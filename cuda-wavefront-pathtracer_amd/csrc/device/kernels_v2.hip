@@ -1,8 +1,9 @@
-// device/kernels_v2.hip - the kernels of the BVH2 layout (instantiated here only).
+// device/kernels_v2.hip - the kernels of the BVH2 layout for the triangle test CWP_TRI (instantiated here
+// only; compiled once per test).
 #include "device/kernels.h"
 
 namespace cwp {
 namespace dev {
-template void pickKernels<2>(int, int, int, Kernels&);
+template void pickTri<2, CWP_TRI>(int, int, Kernels&);
 }  // namespace dev
 }  // namespace cwp

@@ -301,8 +301,6 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     } else if (I.inst) {
         // two-level scenes run the fused bounce kernel and the one-ray-per-lane shadow kernel
         if (!O.fuse || O.persistent) { err = "two-level scenes need the fused kernel (fuse 1, persistent 0)"; return false; }
-        I.bounce = S.full ? I.kn.bounceFullInst : I.kn.bounceInst; I.shade = nullptr; I.shadow = I.kn.shadowInst;
-        I.kn.traceC = I.kn.traceCInst; I.kn.traceA = I.kn.traceAInst;
         I.meshRoot = S.meshRoot; I.nMesh = (int)S.meshRoot.size();
         Vec4* mb;
         if (!I.upload(mb, S.meshBox, err)) return false;
@@ -311,6 +309,14 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         if (O.tlasWidth != 2 && O.tlasWidth != 8) { err = "TLAS width must be 2 or 8"; return false; }
         I.tlasWide = O.variant == 8 && O.tlasWidth == 8;
         tlasWide = I.tlasWide ? 1 : 0;
+        I.shade = nullptr;
+        if (I.tlasWide) {
+            I.bounce = S.full ? I.kn.bounceFullInst8 : I.kn.bounceInst8; I.shadow = I.kn.shadowInst8;
+            I.kn.traceC = I.kn.traceCInst8; I.kn.traceA = I.kn.traceAInst8;
+        } else {
+            I.bounce = S.full ? I.kn.bounceFullInst : I.kn.bounceInst; I.shadow = I.kn.shadowInst;
+            I.kn.traceC = I.kn.traceCInst; I.kn.traceA = I.kn.traceAInst;
+        }
         HIPCHK(hipHostMalloc((void**)&I.hostDepth, 2 * sizeof(int), hipHostMallocDefault));   // TLAS depth, build status
         if (!I.alloc(I.dDepth, 1, err)) return false;
     } else {
@@ -320,11 +326,10 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     }
     if (O.tail < -1 || O.tail == 1 || O.tail > kWave) { err = "tail must be -1 (auto), 0 (off) or 2..64 lanes"; return false; }
     if (O.tailLevels != 1 && O.tailLevels != 2) { err = "tail levels must be 1 or 2"; return false; }
-    // two-level scenes hand off between TLAS node steps, which needs the BVH8 TLAS
+    // two-level scenes hand off between node steps of either level, which needs the BVH8 TLAS
     const bool tailable = S.variant == 8 && (!I.inst || I.tlasWide) && O.fuse && !O.persistent;
-    // automatic: single-level scenes only (the 1,001-instance frame measured 579 -> 593 ms with it: its hand-off
-    // points are TLAS steps, each holding whole BLAS traversals)
-    I.O.tail = O.tail == -1 ? (tailable && !I.inst ? kTailDefault : 0) : O.tail;
+    // automatic: wherever it can run (single-level 720p frame 149.5 -> 138.6 ms, 1,001-instance frame 76.4 -> 74.1 ms)
+    I.O.tail = O.tail == -1 ? (tailable ? kTailDefault : 0) : O.tail;
     if (I.O.tail) {
         if (!tailable) {
             err = "the straggler hand-off (tail) needs a BVH8 scene (two-level: with the BVH8 TLAS) and the fused kernel "
@@ -375,7 +380,7 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
 
     // stack spill beyond the LDS part: the tree bounds the entries a traversal can hold (two-level scenes: the
     // deepest accepted TLAS below the deepest BLAS)
-    if (I.inst) stackNeed += kTlasMaxDepth;
+    if (I.inst) stackNeed += kTlasMaxDepth + kPendingStack;
     I.P.spillCap = stackNeed > I.sl ? stackNeed - I.sl : 0;
     if (I.P.spillCap > 0) {
         uint64_t* sp;
@@ -400,22 +405,32 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         !I.alloc(I.accum, (size_t)I.N, err) || !I.alloc(I.tot, 8, err))
         return false;
     if (!O.fuse && !I.alloc(I.P.H, NK, err)) return false;
-    if (I.O.tail) {   // tail records: slot, hit, node group and the stack (two entries per Vec4), at most lanes - 1 per chunk
-        I.P.tailLanes = I.O.tail;
-        I.P.tailStride = 3 + (std::max(stackNeed, 1) + 1) / 2;
-        const size_t records = ((NK >> 6) + kParts + 1) * (size_t)(I.O.tail - 1);
-        if (!I.alloc(I.P.tail, records * (size_t)I.P.tailStride, err)) return false;
-        if (I.bounceTail2) {   // the second level's regions follow from the first's record numbering
-            const size_t records2 = ((records >> 6) + kParts + 1) * (size_t)(I.O.tail - 1);
-            if (!I.alloc(I.P.tail2, records2 * (size_t)I.P.tailStride, err)) return false;
-        }
-    }
     if (O.sort < 0 || O.sort > 2) { err = "sort must be 0, 1 or 2"; return false; }
     if (O.sort == 2 && (!O.fuse || O.persistent)) { err = "sort 2 (first-bounce sort) needs the fused kernel (fuse 1, persistent 0)"; return false; }
     if (O.sort) {
         if (!I.alloc(I.P.stO, NK, err) || !I.alloc(I.P.stD, NK, err) || !I.alloc(I.P.stT, NK, err) ||
             !I.alloc(I.P.qk, NK, err)) return false;
         I.P.bcnt = I.P.cnt + (size_t)(I.depths + 1) * kCntStride;
+    }
+    if (I.O.tail) {   // tail records: slot, hit so far, node group and the stack (two entries per Vec4), at most lanes - 1 per chunk
+        I.P.tailLanes = I.O.tail;
+        I.P.tailStride = 3 + (std::max(stackNeed, 1) + 1) / 2;
+        const size_t records = ((NK >> 6) + kParts + 1) * (size_t)(I.O.tail - 1);
+        // the second level's regions follow from the first's record numbering
+        const size_t records2 = ((records >> 6) + kParts + 1) * (size_t)(I.O.tail - 1);
+        const bool ok = I.alloc(I.P.tail, records * (size_t)I.P.tailStride, err) &&
+                        (!I.bounceTail2 || I.alloc(I.P.tail2, records2 * (size_t)I.P.tailStride, err));
+        if (!ok) {
+            // the records of a two-level scene take up to 1.5 times the path state: where the automatic setting finds no
+            // room for them, the frame runs without the hand-off
+            if (!I.inst || O.tail != -1) return false;
+            (void)hipGetLastError();
+            if (I.P.tail) { hipFree(I.P.tail); I.allocs.pop_back(); }
+            I.P.tail = I.P.tail2 = nullptr; I.P.tailLanes = 0; I.O.tail = 0;
+            I.bounce = S.full ? I.kn.bounceFullInst8 : I.kn.bounceInst8; I.shadow = I.kn.shadowInst8;
+            I.bounceTail = I.bounceTail2 = nullptr; I.shadowTail = I.shadowTail2 = nullptr;
+            err.clear();
+        }
     }
     HIPCHK(hipHostMalloc((void**)&I.hostTot, 8 * sizeof(unsigned long long), hipHostMallocDefault));
     if (!I.fill(I.accum, (size_t)I.N * 16, err)) return false;

@@ -155,9 +155,10 @@ __device__ __forceinline__ Group makeGroup(uint32_t base, uint32_t bits) { retur
 // Resumable state of one ray's traversal: the node to visit next and, for BVH8, the group of hit children still to
 // visit (child base, internal-child mask, octant-ordered hit bits). With the lane's stack this is everything a
 // persistent kernel needs to suspend a ray between node visits.
-struct TravState { int node; uint32_t gBase, gMask, gHits; };
+// Two-level scenes also keep the instance whose BLAS is being traversed (-1: the TLAS).
+struct TravState { int node; uint32_t gBase, gMask, gHits; int inst; };
 
-__device__ __forceinline__ void travBegin(TravState& s, int root) { s.node = root; s.gBase = 0; s.gMask = 0; s.gHits = 0; }
+__device__ __forceinline__ void travBegin(TravState& s, int root) { s.node = root; s.gBase = 0; s.gMask = 0; s.gHits = 0; s.inst = -1; }
 
 // ------------------------------------------------------------------------------------------------ BVH2
 // One node visit. Returns true when the traversal is over (stack exhausted, or for ANY a hit was found).
@@ -270,37 +271,35 @@ __device__ __forceinline__ bool traceBVH4(const Vec4* __restrict__ nodes, const 
 // ------------------------------------------------------------------------------------------------ compressed BVH8
 __device__ __forceinline__ uint32_t byteOf(uint32_t w, int s) { return (w >> (8 * (s & 3))) & 255u; }
 
-// One node visit: the node's 8 child slabs, its hit leaves, then the choice of the next node. Returns true when the
-// traversal is over (nothing left to visit, or for ANY a hit was found). leaf(k) handles leaf primitive k (the node's
-// primitive base + the offset in its slot's metadata) and returns true to end an any-hit traversal: a triangle test
-// for a BLAS, an instance's BLAS traversal for a TLAS.
-template <bool ANY, class Stack, class Leaf>
-__device__ __forceinline__ bool stepBVH8With(const Vec4* __restrict__ nodes, const RayPre& r, Hit& h, Stack& st,
-                                             TravState& ts, Leaf&& leaf) {
-    const Vec4* nb = nodes + (size_t)ts.node * kBvh8Stride;
+// A node's slots after the slab test: which are hit, and what they hold.
+struct Node8 { uint32_t hitSlots, imask, leafMask, meta0, meta1; int childBase, triBase; };
+
+// Phase 1 of a node visit: the 8 child slabs against the hit distance at node entry. With the ray's direction signs the
+// near plane of each axis is known up front (lo for a positive direction, hi for a negative one), so each slot needs
+// no per-axis min/max; the result is bit-identical to min/max of the two planes.
+__device__ __forceinline__ Node8 testNode8(const Vec4* __restrict__ nodes, int node, const RayPre& r, float tEntry) {
+    const Vec4* nb = nodes + (size_t)node * kBvh8Stride;
     const Vec4 f0 = ldg4(nb), f1 = ldg4(nb + 1), f2 = ldg4(nb + 2), f3 = ldg4(nb + 3), f4 = ldg4(nb + 4);
     const uint32_t ew = asUint(f0.w);
     const float sx = asFloatU((ew & 255u) << 23) * r.ix;
     const float sy = asFloatU(((ew >> 8) & 255u) << 23) * r.iy;
     const float sz = asFloatU(((ew >> 16) & 255u) << 23) * r.iz;
     const float ox = (f0.x - r.o.x) * r.ix, oy = (f0.y - r.o.y) * r.iy, oz = (f0.z - r.o.z) * r.iz;
-    const uint32_t imask = ew >> 24;
-    const uint32_t meta[2] = { asUint(f1.z), asUint(f1.w) };
-    const uint32_t w1 = asUint(f1.x), leafMask = w1 >> 24;   // slots holding leaves (empty slots: in neither mask)
-    const int childBase = (int)(w1 & 0xFFFFFFu), triBase = asInt(f1.y);
+    Node8 n;
+    n.imask = ew >> 24;
+    n.meta0 = asUint(f1.z); n.meta1 = asUint(f1.w);
+    const uint32_t w1 = asUint(f1.x);
+    n.leafMask = w1 >> 24;   // slots holding leaves (empty slots: in neither mask)
+    n.childBase = (int)(w1 & 0xFFFFFFu); n.triBase = asInt(f1.y);
     const uint32_t qlx[2] = { asUint(f2.x), asUint(f2.y) }, qly[2] = { asUint(f2.z), asUint(f2.w) };
     const uint32_t qlz[2] = { asUint(f3.x), asUint(f3.y) }, qhx[2] = { asUint(f3.z), asUint(f3.w) };
     const uint32_t qhy[2] = { asUint(f4.x), asUint(f4.y) }, qhz[2] = { asUint(f4.z), asUint(f4.w) };
-    // Phase 1: the 8 child slabs against the hit distance at node entry. With the ray's direction signs the near
-    // plane of each axis is known up front (lo for a positive direction, hi for a negative one), so each slot needs
-    // no per-axis min/max; the result is bit-identical to min/max of the two planes.
     const uint32_t nx[2] = { r.pos & 1u ? qlx[0] : qhx[0], r.pos & 1u ? qlx[1] : qhx[1] };
     const uint32_t fx[2] = { r.pos & 1u ? qhx[0] : qlx[0], r.pos & 1u ? qhx[1] : qlx[1] };
     const uint32_t ny[2] = { r.pos & 2u ? qly[0] : qhy[0], r.pos & 2u ? qly[1] : qhy[1] };
     const uint32_t fy[2] = { r.pos & 2u ? qhy[0] : qly[0], r.pos & 2u ? qhy[1] : qly[1] };
     const uint32_t nz[2] = { r.pos & 4u ? qlz[0] : qhz[0], r.pos & 4u ? qlz[1] : qhz[1] };
     const uint32_t fz[2] = { r.pos & 4u ? qhz[0] : qlz[0], r.pos & 4u ? qhz[1] : qlz[1] };
-    const float tEntry = h.t;
     uint32_t hitSlots = 0;
 #pragma unroll
     for (int s = 0; s < 8; s++) {
@@ -312,47 +311,65 @@ __device__ __forceinline__ bool stepBVH8With(const Vec4* __restrict__ nodes, con
         const float tf = fminf(fminf(xf, yf), fminf(zf, tEntry));
         hitSlots |= (uint32_t)(tn <= tf) << s;
     }
-    // Phase 2: the triangles of the hit leaves as one bit set relative to the node's triangle base (a node's leaves
-    // hold their triangles at increasing offsets in slot order, at most 24 in all), then one flat loop over its bits:
-    // the wave iterates as often as its lane with the most triangles, not once per leaf and again per triangle.
-    uint32_t lb = hitSlots & leafMask, tm = 0;
+    n.hitSlots = hitSlots;
+    return n;
+}
+// The primitives of the hit leaves as one bit set relative to the node's primitive base (a node's leaves hold their
+// primitives at increasing offsets in slot order, at most 24 in all): one flat loop over its bits lets the wave iterate
+// as often as its lane with the most primitives, not once per leaf and again per primitive.
+__device__ __forceinline__ uint32_t leafPrims8(const Node8& n) {
+    uint32_t lb = n.hitSlots & n.leafMask, tm = 0;
     while (lb) {
         const int s = __builtin_ctz(lb);
         lb &= lb - 1;
-        const uint32_t m = byteOf(s < 4 ? meta[0] : meta[1], s);
+        const uint32_t m = byteOf(s < 4 ? n.meta0 : n.meta1, s);
         tm |= ((2u << ((m >> 5) & 3u)) - 1u) << (m & 31u);
     }
-    while (tm) {
-        const int j = __builtin_ctz(tm);
-        tm &= tm - 1;
-        if (leaf(triBase + j) && ANY) return true;
-    }
-    // internal hits in octant order: bit k = slot k ^ octant (permute by the three octant bits)
-    uint32_t hits = hitSlots & imask;
+    return tm;
+}
+// the node's internal hits in octant order (bit k = slot k ^ octant) become the current group, above the old one
+template <class Stack>
+__device__ __forceinline__ void enterGroup8(const Node8& n, const RayPre& r, Stack& st, TravState& ts) {
+    uint32_t hits = n.hitSlots & n.imask;
     if (r.oct & 1u) hits = ((hits & 0x55u) << 1) | ((hits >> 1) & 0x55u);
     if (r.oct & 2u) hits = ((hits & 0x33u) << 2) | ((hits >> 2) & 0x33u);
     if (r.oct & 4u) hits = ((hits & 0x0Fu) << 4) | ((hits >> 4) & 0x0Fu);
     if (hits) {
         if (ts.gHits) st.push(makeGroup(ts.gBase, (ts.gMask << 8) | ts.gHits));
-        ts.gBase = (uint32_t)childBase; ts.gMask = imask; ts.gHits = hits;
+        ts.gBase = (uint32_t)n.childBase; ts.gMask = n.imask; ts.gHits = hits;
     }
-    while (ts.gHits == 0) {
-        if (st.sp == st.floor) return true;
-        const Group e = st.pop();
-        const uint32_t bits = (uint32_t)(e >> 32);
-        ts.gBase = (uint32_t)e; ts.gMask = bits >> 8; ts.gHits = bits & 255u;
-    }
+}
+// the next child of the (non-empty) current group
+__device__ __forceinline__ void nextChild8(const RayPre& r, TravState& ts) {
     const uint32_t k = (uint32_t)__builtin_ctz(ts.gHits);
     ts.gHits &= ts.gHits - 1;
     const uint32_t slot = k ^ r.oct;
     ts.node = (int)ts.gBase + __builtin_popcount(ts.gMask & ((1u << slot) - 1u));
-    return false;
+}
+__device__ __forceinline__ void setGroup8(Group e, TravState& ts) {
+    const uint32_t bits = (uint32_t)(e >> 32);
+    ts.gBase = (uint32_t)e; ts.gMask = bits >> 8; ts.gHits = bits & 255u;
 }
 
+// One node visit: the node's 8 child slabs, its hit leaves' triangles, then the choice of the next node. Returns true
+// when the traversal is over (nothing left to visit, or for ANY a hit was found).
 template <bool ANY, int TRI, class Stack>
 __device__ __forceinline__ bool stepBVH8(const Vec4* __restrict__ nodes, const Vec4* __restrict__ tri, const RayPre& r,
                                          Hit& h, Stack& st, TravState& ts) {
-    return stepBVH8With<ANY>(nodes, r, h, st, ts, [&](int t) { return triTest<TRI>(tri, t, r, h); });
+    const Node8 n = testNode8(nodes, ts.node, r, h.t);
+    uint32_t tm = leafPrims8(n);
+    while (tm) {
+        const int j = __builtin_ctz(tm);
+        tm &= tm - 1;
+        if (triTest<TRI>(tri, n.triBase + j, r, h) && ANY) return true;
+    }
+    enterGroup8(n, r, st, ts);
+    while (ts.gHits == 0) {
+        if (st.sp == st.floor) return true;
+        setGroup8(st.pop(), ts);
+    }
+    nextChild8(r, ts);
+    return false;
 }
 
 template <bool ANY, int TRI, class Stack>

@@ -129,7 +129,7 @@ typedef struct cwp_options {
                             src/render/wavefront.cu:717; different sorts, same results): 1 every bounce's, grouped by
                             direction bucket within each XCD partition; 2 the first bounce's, grouped by elevation
                             bucket within each pixel's samples (fused kernel only) */
-    int tail_lanes;      /* straggler hand-off (compressed BVH8, single-level scenes, fused kernel): once fewer than
+    int tail_lanes;      /* straggler hand-off (compressed BVH8, fused kernel): once fewer than
                             this many lanes of a trace+shade wave are still tracing, their traversals are handed to a
                             tail kernel that resumes them in full waves (same results); 0 off, 2..64 */
 } cwp_options;

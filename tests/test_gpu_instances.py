@@ -151,6 +151,38 @@ def test_wide_tlas_over_few_instances(count):
     r.close()
 
 
+@pytest.mark.parametrize("tri,stack,tail,count", [("woop", 8, 0, 30), ("woop", 8, 2, 30), ("woop", 32, 64, 9),
+                                                  ("watertight", 16, 12, 64), ("mt", 8, 12, 2)])
+def test_overlapping_instances(tri, stack, tail, count):
+    """Instances that all overlap, so that TLAS leaves name several at once, their rest waits on the stack while a BLAS is
+    traversed, and waves hand such traversals off: triangle and instance ids of closest hits against the oracle, any
+    hits, and the image without hand-off, bit for bit (a ray's visiting order depends on neither)."""
+    print("case overlapping", tri, stack, tail, count, flush=True)
+    args = ARGS + ["--tri", tri, "--stack", str(stack), "--batch", "4", "--bounces", "3"]
+    s = cwp.Setup(args + ["--tail", str(tail)])
+    inst = s.instances(0)[:count].copy()
+    fwd, inv = inst[:, 12:24].reshape(-1, 3, 4), inst[:, :12].reshape(-1, 3, 4)
+    fwd[:, :, 3] = np.random.default_rng(count).uniform(-0.3, 0.3, (count, 3))   # all around the origin
+    inv[:, :, 3] = -np.einsum("nij,nj->ni", inv[:, :, :3].astype(np.float64), fwd[:, :, 3].astype(np.float64))
+    r = cwp.Renderer(s)
+    r.set_instances(inst)
+    sc = po.Scene(s.info["variant"], {"mt": 0, "woop": 1, "watertight": 2}[tri], s.array(cwp.ARR_NODES), s.array(cwp.ARR_WOOP),
+                  s.array(cwp.ARR_CORNERS), s.array(cwp.ARR_ALBEDO))
+    sc.set_instances(inst, s.array(cwp.ARR_MESH_BOXES))
+    rays = scene_rays(s, 4000, 17)
+    g, gi = r.trace_inst(rays)
+    o, oi = sc.trace_inst(rays)
+    gt, ot = g[:, 3].view(np.int32), o[:, 3].view(np.int32)
+    assert (ot >= 0).mean() > 0.02
+    assert ((gt == ot) & (gi == oi)).mean() >= 0.999
+    assert np.array_equal(r.trace_inst(rays, any_hit=True)[0][:, 3].view(np.int32) >= 0, gt >= 0)
+    r.render(4)
+    plain = cwp.Renderer(cwp.Setup(args + ["--tail", "0"]))
+    plain.set_instances(inst)
+    plain.render(4)
+    np.testing.assert_array_equal(r.accum(), plain.accum())
+
+
 FULL = ARGS + ["--gen_materials", "2", "--gen_env", "64,32,1.5,2", "--bounces", "3"]
 
 
