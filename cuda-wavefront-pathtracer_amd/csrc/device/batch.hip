@@ -112,7 +112,7 @@ struct BatchRenderer::Impl {
     bool shadowTail() const { return O.tail && O.full; }
     // the launches of a pass reading table slot s
     void enqueue(int s) {
-        k_pass_begin_jobs<<<1, 64, 0, st>>>(P.cnt, (depths + 1) * kCntStride, dTable[s]);
+        k_pass_begin_jobs<<<1, kPassBegin, 0, st>>>(P.cnt, (depths + 1) * kCntStride, dTable[s]);
         const int gb = O.full ? gridFull : grid;
         for (int depth = 0; depth < depths; depth++) {
             if (O.tail) {   // the hand-off kernel, then its tail (same grid: within the spill area's lanes)
@@ -129,7 +129,7 @@ struct BatchRenderer::Impl {
             }
         }
         k_reduce_jobs<<<redGrid, kWave, 0, st>>>(dTable[s], P.L);
-        k_pass_end<<<1, 64, 0, st>>>(P.cnt, depths, tot);
+        k_pass_end<<<1, kWave, 0, st>>>(P.cnt, depths, 0, tot, nullptr);
     }
     // the launches of a rolling step reading step-table slot s (step parity = s & 1)
     void enqueueStep(int s, int step) {
@@ -257,10 +257,10 @@ bool BatchRenderer::init(const BatchOptions& O, std::string& err) {
     if (!I.alloc(I.P.O[0], n, err) || !I.alloc(I.P.D[0], n, err) || !I.alloc(I.P.T[0], n, err) ||
         !I.alloc(I.P.O[1], n, err) || !I.alloc(I.P.D[1], n, err) || !I.alloc(I.P.T[1], n, err) || !I.alloc(I.P.L, n, err) ||
         !I.alloc(I.P.sO, n, err) || !I.alloc(I.P.sD, n, err) ||
-        !I.alloc(I.P.sC, n, err) || !I.alloc(I.P.cnt, (size_t)(I.depths + 1) * kCntStride, err) || !I.alloc(I.tot, 8, err))
+        !I.alloc(I.P.sC, n, err) || !I.alloc(I.P.cnt, (size_t)(I.depths + 1) * kCntStride, err) || !I.alloc(I.tot, kTot, err))
         return false;
     HIPCHK(hipHostMalloc((void**)&I.hostTot, 8 * sizeof(unsigned long long), hipHostMallocDefault));
-    if (!I.fill(I.tot, 8 * sizeof(unsigned long long), 0u, err) || !I.ensureTail(err)) return false;
+    if (!I.fill(I.tot, kTot * sizeof(unsigned long long), 0u, err) || !I.ensureTail(err)) return false;
     for (int k = 0; k < kTableSlots; k++) {
         if (!I.alloc(I.dTable[k], 1, err)) return false;
         HIPCHK(hipHostMalloc((void**)&I.hTable[k], sizeof(DevJobTable), hipHostMallocDefault));

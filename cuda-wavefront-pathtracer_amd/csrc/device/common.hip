@@ -11,6 +11,7 @@ __global__ void __launch_bounds__(kBlock) k_shade(DevScene S, DevPaths P, const 
     const int lane = laneId();
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
     int* cnt = P.cnt + depth * kCntStride;
+    stamp(cnt, kCStampShade);
     const int n = ctrv(cnt, part, kCQueue);
     const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
     const int outStart = partStart(cnt, part);
@@ -52,6 +53,7 @@ __global__ void __launch_bounds__(kSortBlock) k_qcount(DevPaths P, int depth) {
     __shared__ int h[kBuckets];
     const int t = (int)threadIdx.x;
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    stamp(P.cnt + depth * kCntStride, kCStampSort);
     int start, n;
     sortRange(P, depth, part, start, n);
     if (t < kBuckets) h[t] = 0;
@@ -122,6 +124,7 @@ __global__ void __launch_bounds__(kFirstTile) k_qsort_first(DevPaths P) {
     const int t = (int)threadIdx.x;
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
     const int* cnt0 = P.cnt;
+    stamp(P.cnt, kCStampSort);
     const int start = partStart(cnt0, part), n = ctrv(cnt0, part, kCQueue);
     int* queue = ctr(P.cnt + kCntStride, part, kCQueue);
     for (int tile = lw; tile * kFirstTile < n; tile += nw) {   // block-uniform bound: every thread meets the barriers
@@ -148,29 +151,52 @@ __global__ void k_pass_begin(int* cnt, int words, long long NK) { passBegin(cnt,
 // a batched pass: the path count comes from the pass's job table on the device
 __global__ void k_pass_begin_jobs(int* cnt, int words, const DevJobTable* T) { passBegin(cnt, words, T->paths); }
 
-// per-pass totals: [0] closest rays, [1] shadow rays, [2] misses, [3] unoccluded, [4] continuations,
-// [5] camera-ray misses
-__global__ void k_pass_end(const int* cnt, int depths, unsigned long long* tot) {
-    if (threadIdx.x != 0) return;
-    unsigned long long a = 0, b = 0, m = 0, u = 0, c = 0, m0 = 0;
-    for (int x = 0; x < kParts; x++) m0 += (unsigned)ctrv(cnt, x, kCMiss);
-    for (int d = 0; d < depths; d++) {
+// Per-pass totals: [0] closest rays, [1] shadow rays, [2] misses, [3] unoccluded, [4] continuations, [5] camera-ray
+// misses, then the launches' times in device-clock ticks: [6] trace+shade, [7] the tails' part of it and of the shadow
+// launches, [8] the shade launches' part, [9] shadow, [10] sort. One wave, a lane per depth (on one lane the dependent
+// loads of ten depths took 30 us).
+__global__ void __launch_bounds__(kWave) k_pass_end(const int* cnt, int depths, int first, unsigned long long* tot, unsigned long long* host) {
+    unsigned long long v[kTot] = {};
+    for (int d = (int)threadIdx.x; d < depths; d += kWave) {
         const int* cd = cnt + d * kCntStride;
-        unsigned long long q = 0;
+        unsigned q = 0, b = 0, m = 0, u = 0;
         for (int x = 0; x < kParts; x++) {
             q += (unsigned)ctrv(cd, x, kCQueue); b += (unsigned)ctrv(cd, x, kCShadow);
             m += (unsigned)ctrv(cd, x, kCMiss); u += (unsigned)ctrv(cd, x, kCUnocc);
         }
-        a += q; if (d > 0) c += q;
+        v[0] += q; v[1] += b; v[2] += m; v[3] += u;
+        if (d > 0) v[4] += q; else v[5] += m;
+        auto at = [&](const int* c, int word) { return *(const unsigned long long*)(c + word); };
+        const unsigned long long bounce = at(cd, kCStampBounce), tail = at(cd, kCStampTail), shade = at(cd, kCStampShade);
+        const unsigned long long shadow = at(cd, kCStampShadow), stail = at(cd, kCStampShadowTail), sort = at(cd, kCStampSort);
+        // the next depth's launch, or the reduction's stamp in the block after the last depth
+        const unsigned long long next = d + 1 < depths && at(cd + kCntStride, kCStampBounce) ? at(cd + kCntStride, kCStampBounce)
+                                                                                             : at(cnt + depths * kCntStride, kCStampBounce);
+        const unsigned long long bEnd = shadow ? shadow : next, sEnd = sort ? sort : next;
+        if (bounce) v[6] += bEnd - bounce;
+        if (tail) v[7] += (shade ? shade : bEnd) - tail;
+        if (stail) v[7] += sEnd - stail;
+        if (shade) v[8] += bEnd - shade;
+        if (shadow) v[9] += sEnd - shadow;
+        if (sort) v[10] += next - sort;
     }
-    tot[0] += a; tot[1] += b; tot[2] += m; tot[3] += u; tot[4] += c; tot[5] += m0;
+    for (int k = 0; k < kTot; k++) {
+        for (int o = 1; o < kWave; o <<= 1) v[k] += __shfl_xor(v[k], o);
+        if (threadIdx.x == 0) {
+            if (!first) v[k] += tot[k];
+            tot[k] = v[k];
+            if (host) host[k] = v[k];
+        }
+    }
 }
 
 // accum[pix] += sum over the K samples of the pass (path ids pix*K .. pix*K + K-1), in sample order. One wave per 64
 // pixels: the K samples of a pixel are contiguous, so the wave loads chunks of 16 samples of 4 pixels per instruction
 // (4 runs of 256 B) into LDS, then each lane adds its pixel's samples in order.
 constexpr int kRedChunk = 16;
-__global__ void __launch_bounds__(kWave) k_reduce(const Vec4* __restrict__ L, Vec4* __restrict__ accum, int N, int K) {
+__global__ void __launch_bounds__(kWave) k_reduce(const Vec4* __restrict__ L, Vec4* __restrict__ accum, int N, int K, int clear,
+                                                  unsigned long long* endStamp) {
+    if (endStamp && blockIdx.x == 0 && threadIdx.x == 0) *endStamp = wall_clock64();
     __shared__ float buf[kWave][3 * kRedChunk + 1];   // +1: rows 49 words apart, no bank conflicts between lanes
     const int lane = laneId();
     for (int p0 = blockIdx.x * kWave; p0 < N; p0 += gridDim.x * kWave) {
@@ -189,7 +215,7 @@ __global__ void __launch_bounds__(kWave) k_reduce(const Vec4* __restrict__ L, Ve
             __syncthreads();
         }
         const int pix = p0 + lane;
-        if (pix < N) { Vec4 a = accum[pix]; a.x += r; a.y += g; a.z += b; accum[pix] = a; }
+        if (pix < N) { Vec4 a = clear ? v4(0.f, 0.f, 0.f, 0.f) : accum[pix]; a.x += r; a.y += g; a.z += b; accum[pix] = a; }
     }
 }
 

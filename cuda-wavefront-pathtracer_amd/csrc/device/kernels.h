@@ -49,6 +49,10 @@ constexpr int kCIn = 4, kCMissCam = 5;
 constexpr int kCTail = 6, kCShadowTail = 7;   // ... and [kCShadowTail] the shadow kernel's
 // [kCTail2] / [kCShadowTail2]: traversals the first tail kernels handed on to the second ones
 constexpr int kCTail2 = 8, kCShadowTail2 = 9;
+// Device-clock stamps (64 bits each) in partition 0's line: when the depth's first trace+shade, tail, shade, shadow,
+// shadow-tail and sort launch began (0: no such launch). A launch's time is the next stamp minus its own (k_pass_end).
+// An event record between two launches costs 6-10 us of idle GPU, four of them per depth 0.32 ms of a ten-depth frame.
+constexpr int kCStampBounce = 12, kCStampTail = 14, kCStampShade = 16, kCStampShadow = 18, kCStampShadowTail = 20, kCStampSort = 22;
 
 // Lights and materials of the full integrator (device pointers; null / 0 for the legacy integrator)
 struct DevLights {
@@ -422,6 +426,11 @@ __device__ __forceinline__ int waveAppend(uint64_t mask, int* counter) {
     return base + rank;
 }
 
+// the launch's start into stamp `word` of its depth's counter block (workgroups start in order: the first one's start)
+__device__ __forceinline__ void stamp(int* cnt, int word) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *(unsigned long long*)(cnt + word) = wall_clock64();
+}
+
 // adds a wave-uniform count to *counter once per wave (nothing when it is zero)
 __device__ __forceinline__ void waveAdd(int count, int* counter) {
     if (count && laneId() == 0) atomicAdd(counter, count);
@@ -702,6 +711,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce(DevScene S, DevPaths P
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
     int* cnt = P.cnt + depth * kCntStride;
+    stamp(cnt, kCStampBounce);
     const int n = ctrv(cnt, part, kCQueue);
     const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
     const int outStart = partStart(cnt, part);
@@ -747,6 +757,7 @@ __global__ void __launch_bounds__(kFirstTile, WAVES) k_bounce_first(DevScene S, 
                          (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
     const int part = (int)(blockIdx.x % kParts), lb = (int)(blockIdx.x / kParts), nb = (int)(gridDim.x / kParts);
     int* cnt = P.cnt;
+    stamp(cnt, kCStampBounce);
     const int n = ctrv(cnt, part, kCQueue);
     const int start = partStart(cnt, part);   // the depth-0 slots and the depth-1 queue of partition x start here
     int* queue = ctr(cnt + kCntStride, part, kCQueue);
@@ -790,6 +801,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_tail(DevScene S, DevPa
     LaneStack<Group, SL> st{ (LdsPtr<Group>)(lds + threadIdx.x), (Group*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
     int* cnt = P.cnt + depth * kCntStride;
+    if (LEVEL == 1) stamp(cnt, kCStampTail);
     const int nt = ctrv(cnt, part, LEVEL == 1 ? kCTail : kCTail2);
     const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
     const int outStart = partStart(cnt, part);
@@ -829,7 +841,8 @@ __global__ void __launch_bounds__(kBlock, 8) k_trace_paths(DevScene S, DevPaths 
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
-    const int* cnt = P.cnt + depth * kCntStride;
+    int* cnt = P.cnt + depth * kCntStride;
+    stamp(cnt, kCStampBounce);
     const int n = ctrv(cnt, part, kCQueue);
     const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
     int i = -1;                       // queue slot of this lane's ray, -1 = idle
@@ -882,6 +895,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_refill(DevScene S, Dev
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
     int* cnt = P.cnt + depth * kCntStride;
+    stamp(cnt, kCStampBounce);
     const int n = ctrv(cnt, part, kCQueue);
     const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
     const int outStart = partStart(cnt, part);
@@ -960,6 +974,7 @@ __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow(DevSce
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
     int* cnt = P.cnt + depth * kCntStride;
+    stamp(cnt, kCStampShadow);
     const int n = ctrv(cnt, part, kCShadow);
     const int start = partStart(cnt, part);
     int unocc = 0;
@@ -998,6 +1013,7 @@ __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow_tail(D
     LaneStack<Group, SL> st{ (LdsPtr<Group>)(lds + threadIdx.x), (Group*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
     int* cnt = P.cnt + depth * kCntStride;
+    if (LEVEL == 1) stamp(cnt, kCStampShadowTail);
     const int nt = ctrv(cnt, part, LEVEL == 1 ? kCShadowTail : kCShadowTail2);
     const int start = partStart(cnt, part);
     const size_t first1 = tailFirst(start, part, P.tailLanes), first2 = tailFirst(first1, part, P.tailLanes);
@@ -1036,6 +1052,7 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_refill(DevScene S, DevPath
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
     const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
     int* cnt = P.cnt + depth * kCntStride;
+    stamp(cnt, kCStampShadow);
     const int n = ctrv(cnt, part, kCShadow);
     const int start = partStart(cnt, part);
     int k = -1;                       // shadow-queue entry of this lane's ray, -1 = idle
@@ -1708,6 +1725,7 @@ void pickKernels(int tri, int sl, int waves, Kernels& k) {
 
 // layout-independent kernels (device/common.hip)
 __global__ void k_shade(DevScene S, DevPaths P, const FrameParams* __restrict__ Fp, int depth, int smpBase, int K);
+constexpr int kPassBegin = 1024;   // its workgroup (one; 64 threads took 8 us to clear a ten-depth frame's counters)
 __global__ void k_pass_begin(int* cnt, int words, long long NK);
 // continuation sort of the depth-(depth + 1) queue (P.qs, P.qk) into P.q[(depth + 1) & 1], per partition: bucket
 // sizes, then the scatter. Grids of kSortBlock-thread workgroups, a multiple of kParts.
@@ -1715,8 +1733,12 @@ constexpr int kSortBlock = 256, kSortPer = 16, kSortTile = kSortBlock * kSortPer
 __global__ void k_qcount(DevPaths P, int depth);
 __global__ void k_qscatter(DevPaths P, int depth);
 __global__ void k_qsort_first(DevPaths P);
-__global__ void k_pass_end(const int* cnt, int depths, unsigned long long* tot);
-__global__ void k_reduce(const Vec4* __restrict__ L, Vec4* __restrict__ accum, int N, int K);
+// The pass's counters and times added to tot (first: replacing it); with host, the totals so far go there too (pinned).
+// kTotClock of them are ticks of the device clock: trace+shade, tail, shade, shadow, sort launches.
+constexpr int kTotCounts = 6, kTotClock = 5, kTot = kTotCounts + kTotClock;
+__global__ void k_pass_end(const int* cnt, int depths, int first, unsigned long long* tot, unsigned long long* host);
+// clear: the sums replace accum instead of adding to it; endStamp (or null): set to the launch's start
+__global__ void k_reduce(const Vec4* __restrict__ L, Vec4* __restrict__ accum, int N, int K, int clear, unsigned long long* endStamp);
 __global__ void k_fill(uint32_t* p, size_t words, uint32_t v);
 // per triangle of a scene's corner array: (cross(e1, e2), material id bits of the second corner)
 __global__ void k_tri_geo(const Vec4* __restrict__ verts, int nt, Vec4* __restrict__ geo);

@@ -29,7 +29,7 @@ struct RenderOptions {
     int stackLds = 16;      // LDS traversal-stack entries per lane (8, 16 or 32); deeper entries spill to HBM
     int blocksPerCU = 0;    // persistent grid: workgroups per CU (0 = occupancy limit)
     int bounceWaves = 8;    // trace+shade kernel: register budget for at least this many waves per SIMD (1, 6 or 8)
-    int timeKernels = 1;    // per-launch hipEvent timing of the trace/shadow kernels
+    int timeKernels = 1;    // per-launch device-clock timing of the trace/shadow kernels
     int fuse = 1;           // 1: trace and shade in one kernel; 0: a closest-hit trace kernel, then a shade kernel
     int persistent = 0;     // 1: split kernels whose waves refill idle lanes with new rays mid-traversal (implies fuse 0)
     int shadowRefill = 0;   // shadow kernel: 1 = refill idle lanes mid-traversal, 0 = one ray per lane per round

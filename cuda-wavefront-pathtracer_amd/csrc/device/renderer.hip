@@ -113,7 +113,7 @@ struct Renderer::Impl {
     int N = 0, K = 1, NK = 0, depths = 0, sl = 16;
     hipStream_t st = nullptr;
     hipEvent_t f0 = nullptr, f1 = nullptr;
-    std::vector<hipEvent_t> evs; size_t evUsed = 0;
+    double clockMs = 1e-5;        // milliseconds per tick of the device clock (k_pass_end's times)
     DevScene S{};
     DevPaths P{};
     Vec4* accum = nullptr;
@@ -162,10 +162,6 @@ struct Renderer::Impl {
     }
     // pass counters: kCntStride per depth (+1), then the continuation sort's bucket counters per depth
     size_t counterWords() const { return (size_t)(depths + 1) * kCntStride + (O.sort ? (size_t)depths * kSortWords : 0); }
-    hipEvent_t nextEvent() {
-        if (evUsed == evs.size()) { hipEvent_t e; if (hipEventCreate(&e) != hipSuccess) return nullptr; evs.push_back(e); }
-        return evs[evUsed++];
-    }
     bool fill(void* p, size_t bytes, std::string& err) {
         size_t words = bytes / 4;
         int g = (int)std::min<size_t>((words + 255) / 256, 4096);
@@ -191,7 +187,6 @@ Renderer::~Renderer() {
     if (p_->hostDepth) hipHostFree(p_->hostDepth);
     if (p_->tl0) hipEventDestroy(p_->tl0);
     if (p_->tl1) hipEventDestroy(p_->tl1);
-    for (hipEvent_t e : p_->evs) hipEventDestroy(e);
     if (p_->f0) hipEventDestroy(p_->f0);
     if (p_->f1) hipEventDestroy(p_->f1);
     if (p_->hostTot) hipHostFree(p_->hostTot);
@@ -402,7 +397,7 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         !I.alloc(I.P.O[1], NK, err) || !I.alloc(I.P.D[1], NK, err) || !I.alloc(I.P.T[1], NK, err) ||
         !I.alloc(I.P.L, NK, err) || !I.alloc(I.P.sO, NK, err) ||
         !I.alloc(I.P.sD, NK, err) || !I.alloc(I.P.sC, NK, err) || !I.alloc(I.P.cnt, I.counterWords(), err) ||
-        !I.alloc(I.accum, (size_t)I.N, err) || !I.alloc(I.tot, 8, err))
+        !I.alloc(I.accum, (size_t)I.N, err) || !I.alloc(I.tot, kTot, err))
         return false;
     if (!O.fuse && !I.alloc(I.P.H, NK, err)) return false;
     if (O.sort < 0 || O.sort > 2) { err = "sort must be 0, 1 or 2"; return false; }
@@ -432,7 +427,9 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
             err.clear();
         }
     }
-    HIPCHK(hipHostMalloc((void**)&I.hostTot, 8 * sizeof(unsigned long long), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void**)&I.hostTot, kTot * sizeof(unsigned long long), hipHostMallocDefault));
+    int clockKHz = 0;
+    if (hipDeviceGetAttribute(&clockKHz, hipDeviceAttributeWallClockRate, 0) == hipSuccess && clockKHz > 0) I.clockMs = 1.0 / clockKHz;
     if (!I.fill(I.accum, (size_t)I.N * 16, err)) return false;
     HIPCHK(hipStreamSynchronize(I.st));
     size_t free1 = 0;
@@ -458,64 +455,41 @@ bool Renderer::render(int spp, int sBase, bool clear, FrameStats& S, std::string
     if (I.inst && I.full && I.numEmInst > 0 && !I.emSet) { err = "two-level scene: set the emitters of a frame first"; return false; }
     if (sBase < 0) { err = "sample base must be >= 0"; return false; }
     S = FrameStats();
-    I.evUsed = 0;
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> bounceEv, shadeEv, shadowEv, sortEv, tailEv;
     const bool timed = I.O.timeKernels && !I.O.graph;
-    // the frame's launches: clears (by kernels, never memset nodes), then per pass the counter reset, trace+shade
-    // and shadow per bounce, the reduction and the totals
+    // the frame's launches: per pass the counter reset, trace+shade and shadow per bounce, the reduction (which also
+    // clears the sums) and the totals (by kernels, never memset nodes)
     auto enqueue = [&]() -> bool {
-        if (clear && !I.fill(I.accum, (size_t)I.N * 16, err)) return false;
-        if (!I.fill(I.tot, 8 * sizeof(unsigned long long), err)) return false;
         const int words = (int)I.counterWords();
+        unsigned long long* endStamp = (unsigned long long*)(I.P.cnt + (size_t)I.depths * kCntStride + kCStampBounce);
         for (int s = sBase; s < sBase + spp; s += I.K) {
-            k_pass_begin<<<1, 64, 0, I.st>>>(I.P.cnt, words, I.NK);
+            const int first = s == sBase ? 1 : 0;
+            k_pass_begin<<<1, kPassBegin, 0, I.st>>>(I.P.cnt, words, I.NK);
             // first-bounce sort: the depth-0 launch stages its continuations, the later ones append directly
             DevPaths P0 = I.P, Pn = I.P;
             if (I.O.sort == 2) { P0.firstSort = I.bounceFirst ? 0 : 1; Pn.qk = nullptr; P0.qk = I.bounceFirst ? nullptr : P0.qk; }
             for (int depth = 0; depth < I.depths; depth++) {
-                hipEvent_t a = nullptr, b = nullptr;
-                if (timed) { a = I.nextEvent(); b = I.nextEvent(); HIPCHK(hipEventRecord(a, I.st)); }
-                const bool first = depth == 0 && I.bounceFirst;   // depth 0 with the first-bounce sort fused in
-                if (first) I.bounceFirst<<<I.gridFirst, kFirstTile, 0, I.st>>>(I.S, P0, I.dF, s, I.K);
-                else I.bounce<<<I.gridBounce, kBlock, 0, I.st>>>(I.S, depth == 0 ? P0 : Pn, I.dF, depth, s, I.K);
-                if (I.bounceTail && !first) {
-                    if (timed) { hipEvent_t c = I.nextEvent(); HIPCHK(hipEventRecord(c, I.st)); tailEv.push_back({ c, nullptr }); }
-                    I.bounceTail<<<I.gridTail, kBlock, 0, I.st>>>(I.S, depth == 0 ? P0 : Pn, I.dF, depth, s, I.K);
-                    if (I.bounceTail2) I.bounceTail2<<<I.gridTail, kBlock, 0, I.st>>>(I.S, depth == 0 ? P0 : Pn, I.dF, depth, s, I.K);
+                if (depth == 0 && I.bounceFirst) {   // depth 0 with the first-bounce sort fused in
+                    I.bounceFirst<<<I.gridFirst, kFirstTile, 0, I.st>>>(I.S, P0, I.dF, s, I.K);
+                } else {
+                    const DevPaths& Pd = depth == 0 ? P0 : Pn;
+                    I.bounce<<<I.gridBounce, kBlock, 0, I.st>>>(I.S, Pd, I.dF, depth, s, I.K);
+                    if (I.bounceTail) I.bounceTail<<<I.gridTail, kBlock, 0, I.st>>>(I.S, Pd, I.dF, depth, s, I.K);
+                    if (I.bounceTail2) I.bounceTail2<<<I.gridTail, kBlock, 0, I.st>>>(I.S, Pd, I.dF, depth, s, I.K);
                 }
-                if (I.shade) {
-                    if (timed) { hipEvent_t c = I.nextEvent(); HIPCHK(hipEventRecord(c, I.st)); shadeEv.push_back({ c, nullptr }); }
-                    I.shade<<<I.gridShade, kBlock, 0, I.st>>>(I.S, I.P, I.dF, depth, s, I.K);
-                }
-                if (timed) {
-                    HIPCHK(hipEventRecord(b, I.st)); bounceEv.push_back({ a, b });
-                    if (I.shade) shadeEv.back().second = b;
-                    if (I.bounceTail && !first) tailEv.back().second = b;
-                }
-                if (timed) { a = I.nextEvent(); b = I.nextEvent(); HIPCHK(hipEventRecord(a, I.st)); }
+                if (I.shade) I.shade<<<I.gridShade, kBlock, 0, I.st>>>(I.S, I.P, I.dF, depth, s, I.K);
                 I.shadow<<<I.gridShadow, kBlock, 0, I.st>>>(I.S, I.P, depth);
-                if (I.shadowTail) {
-                    if (timed) { hipEvent_t c = I.nextEvent(); HIPCHK(hipEventRecord(c, I.st)); tailEv.push_back({ c, nullptr }); }
-                    I.shadowTail<<<I.gridShadowTail, kBlock, 0, I.st>>>(I.S, I.P, depth);
-                    if (I.shadowTail2) I.shadowTail2<<<I.gridShadowTail, kBlock, 0, I.st>>>(I.S, I.P, depth);
-                }
-                if (timed) {
-                    HIPCHK(hipEventRecord(b, I.st)); shadowEv.push_back({ a, b });
-                    if (I.shadowTail) tailEv.back().second = b;
-                }
+                if (I.shadowTail) I.shadowTail<<<I.gridShadowTail, kBlock, 0, I.st>>>(I.S, I.P, depth);
+                if (I.shadowTail2) I.shadowTail2<<<I.gridShadowTail, kBlock, 0, I.st>>>(I.S, I.P, depth);
                 if (I.O.sort == 2 && !I.bounceFirst && depth == 0 && depth + 1 < I.depths) {
-                    if (timed) { a = I.nextEvent(); b = I.nextEvent(); HIPCHK(hipEventRecord(a, I.st)); }
                     k_qsort_first<<<I.gridSort, kFirstTile, 0, I.st>>>(P0);
-                    if (timed) { HIPCHK(hipEventRecord(b, I.st)); sortEv.push_back({ a, b }); }
                 } else if (I.O.sort == 1 && depth + 1 < I.depths) {
-                    if (timed) { a = I.nextEvent(); b = I.nextEvent(); HIPCHK(hipEventRecord(a, I.st)); }
                     k_qcount<<<I.gridSort, kSortBlock, 0, I.st>>>(I.P, depth);
                     k_qscatter<<<I.gridSort, kSortBlock, 0, I.st>>>(I.P, depth);
-                    if (timed) { HIPCHK(hipEventRecord(b, I.st)); sortEv.push_back({ a, b }); }
                 }
+                if (timed) { S.bounceLaunches++; S.shadowLaunches++; }
             }
-            k_reduce<<<std::min((I.N + kWave - 1) / kWave, 16384), kWave, 0, I.st>>>(I.P.L, I.accum, I.N, I.K);
-            k_pass_end<<<1, 64, 0, I.st>>>(I.P.cnt, I.depths, I.tot);
+            k_reduce<<<std::min((I.N + kWave - 1) / kWave, 16384), kWave, 0, I.st>>>(I.P.L, I.accum, I.N, I.K, clear && first ? 1 : 0, endStamp);
+            k_pass_end<<<1, kWave, 0, I.st>>>(I.P.cnt, I.depths, first, I.tot, s + I.K < sBase + spp ? nullptr : I.hostTot);
         }
         HIPCHK(hipGetLastError());
         return true;
@@ -542,17 +516,15 @@ bool Renderer::render(int spp, int sBase, bool clear, FrameStats& S, std::string
         if (!enqueue()) return false;
     }
     HIPCHK(hipEventRecord(I.f1, I.st));
-    HIPCHK(hipMemcpyAsync(I.hostTot, I.tot, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, I.st));
-    HIPCHK(hipEventSynchronize(I.f1));
     HIPCHK(hipStreamSynchronize(I.st));
     float ms = 0;
     HIPCHK(hipEventElapsedTime(&ms, I.f0, I.f1));
     S.frameMs = ms;
-    for (auto& e : bounceEv) { HIPCHK(hipEventElapsedTime(&ms, e.first, e.second)); S.bounceMs += ms; S.bounceLaunches++; }
-    for (auto& e : shadowEv) { HIPCHK(hipEventElapsedTime(&ms, e.first, e.second)); S.shadowMs += ms; S.shadowLaunches++; }
-    for (auto& e : shadeEv) { HIPCHK(hipEventElapsedTime(&ms, e.first, e.second)); S.shadeMs += ms; }
-    for (auto& e : sortEv) { HIPCHK(hipEventElapsedTime(&ms, e.first, e.second)); S.sortMs += ms; }
-    for (auto& e : tailEv) { HIPCHK(hipEventElapsedTime(&ms, e.first, e.second)); S.tailMs += ms; }
+    if (timed) {
+        S.bounceMs = (double)I.hostTot[6] * I.clockMs; S.tailMs = (double)I.hostTot[7] * I.clockMs;
+        S.shadeMs = (double)I.hostTot[8] * I.clockMs; S.shadowMs = (double)I.hostTot[9] * I.clockMs;
+        S.sortMs = (double)I.hostTot[10] * I.clockMs;
+    }
     S.traceMs = I.O.timeKernels ? S.bounceMs + S.shadowMs : S.frameMs;
     S.rays = (double)I.hostTot[0]; S.shadowRays = (double)I.hostTot[1];
     S.missRays = (double)I.hostTot[2]; S.unoccluded = (double)I.hostTot[3]; S.contRays = (double)I.hostTot[4];

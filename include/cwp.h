@@ -123,7 +123,7 @@ typedef struct cwp_options {
     int stack_lds;       /* LDS traversal-stack entries per lane: 8, 16 or 32 (deeper entries spill to HBM) */
     int blocks_per_cu;   /* workgroups per CU of the persistent grids (0 = occupancy limit) */
     int bounce_waves;    /* fused kernel register budget: at least this many waves per SIMD (1, 6 or 8) */
-    int time_kernels;    /* per-launch event timing (t_bounce_ms, t_shade_ms, t_shadow_ms) */
+    int time_kernels;    /* per-launch device-clock timing (t_bounce_ms, t_shade_ms, t_shadow_ms) */
     int graph;           /* 1: each frame replays a captured HIP graph (per-launch timing off) */
     int sort;            /* continuations reordered before they are traced (reference option --sort,
                             src/render/wavefront.cu:717; different sorts, same results): 1 every bounce's, grouped by

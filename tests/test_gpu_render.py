@@ -370,3 +370,23 @@ def test_straggler_hand_off_rejects_unsupported_schedules():
                    "--tlas", "bvh2", "--tail", "8"])
     with pytest.raises(cwp.CwpError):   # the hand-off resumes BVH8 TLAS steps
         cwp.Renderer(s)
+
+
+@pytest.mark.parametrize("extra,passes", [([], 1), (["--sort", "1"], 2), (["--sort", "2"], 1), (["--fuse", "0"], 3),
+                                          (["--bounces", "0", "--tail", "12"], 2), (["--bounces", "64"], 1)])
+def test_launch_times_and_totals_over_passes(extra, passes):
+    """The launches' times (device-clock stamps) make up the frame's; the image and the ray counts of several passes in
+    one call are those of one call per pass, the first of which clears the sums, whatever they held."""
+    print("case", extra, passes, flush=True)
+    args = ["--gen", "terrain", "--gen_grid", "60", "--width", "97", "--height", "61", "--batch", "4", "--bounces", "4"] + extra
+    r = cwp.Renderer(cwp.Setup(args))
+    r.render(4, sample_base=100)   # what the clear has to remove
+    st = r.render(4 * passes)
+    img = r.accum()
+    parts = st["t_bounce_ms"] + st["t_shadow_ms"] + st["t_sort_ms"]
+    assert 0.3 * st["t_frame_ms"] < parts <= st["t_frame_ms"] and st["t_trace_ms"] == st["t_bounce_ms"] + st["t_shadow_ms"]
+    assert st["t_tail_ms"] + st["t_shade_ms"] <= parts
+    one = [r.render(4, sample_base=4 * k, clear=k == 0) for k in range(passes)]
+    np.testing.assert_array_equal(img, r.accum())
+    for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
+        assert st[key] == sum(s[key] for s in one), key
