@@ -49,6 +49,8 @@ constexpr int kCIn = 4, kCMissCam = 5;
 constexpr int kCTail = 6, kCShadowTail = 7;   // ... and [kCShadowTail] the shadow kernel's
 // [kCTail2] / [kCShadowTail2]: traversals the first tail kernels handed on to the second ones
 constexpr int kCTail2 = 8, kCShadowTail2 = 9;
+// [kCNext] whole-path kernel: paths of the partition handed out
+constexpr int kCNext = 10;
 // Device-clock stamps (64 bits each) in partition 0's line: when the depth's first trace+shade, tail, shade, shadow,
 // shadow-tail and sort launch began (0: no such launch). A launch's time is the next stamp minus its own (k_pass_end).
 // An event record between two launches costs 6-10 us of idle GPU, four of them per depth 0.32 ms of a ten-depth frame.
@@ -1101,6 +1103,84 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_refill(DevScene S, DevPath
     waveAdd(sum, ctr(cnt, part, kCUnocc));
 }
 
+// Whole paths in one launch: each lane carries a path from its camera ray to its end, tracing, shading and testing the
+// shadow ray of one depth per round, and takes a new path when its own has ended (once pathRefill lanes of the wave
+// are idle). Nothing is queued between depths. For frames with few paths in flight: there a launch per depth holds less
+// work than its latency (the longest ray of the depth, then the tails, then the shadow ray's), six launches per depth;
+// here a wave waits only for its own lanes (321x181, 1 sample, 4 bounces: 0.98 ms of kernels in 36 launches before).
+// Paths are handed out per partition (the band of the image whose scene data
+// this XCD's L2 holds); a wave whose partition has none left goes on with the next one's, so no XCD idles on a
+// partition of short paths. A path's arithmetic, and the order of its additions to L, are those of the queue kernels.
+// Idle lanes take new paths together once this many are idle: 32 against 16 is 2-3 % faster over one level (a refilled
+// lane's camera ray keeps the whole wave a round longer), 1 % slower over two.
+constexpr int pathRefill(int inst) { return inst == kOneLevel ? 32 : 16; }
+// Register budget: 5 waves per SIMD hold the legacy kernels without spills (96 VGPRs), the full integrator needs 4 (128);
+// 6 waves with spills measured 3 % and 10-20 % slower.
+template <int V, int TRI, int SL, int INST, bool FULL>
+__global__ void __launch_bounds__(kBlock, FULL ? 4 : 5) k_path(DevScene S, DevPaths P, const FrameParams* __restrict__ Fp, int smpBase, int K) {
+    const FrameParams& F = *Fp;
+    using E = typename StackEntry<V>::type;
+    __shared__ E lds[SL > 0 ? SL * kBlock : 1];
+    const int gtid = blockIdx.x * kBlock + threadIdx.x;
+    LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
+    int* cnt = P.cnt;   // every depth's counts go to the first block, continuations to the second
+    stamp(cnt, kCStampBounce);
+    const int own = (int)(blockIdx.x % kParts);
+    int part = own, left = kParts;   // wave-uniform: the partition paths are taken from, partitions not yet used up
+    int i = -1, depth = 0;           // this lane's path id (-1: idle) and the depth of its ray
+    Vec3 o, d, T;
+    float lastPdf = 0.f;
+    o = d = T = v3(0.f, 0.f, 0.f);
+    int nShadow = 0, nMiss = 0, nMissCam = 0, nUnocc = 0, nCont = 0;   // wave-uniform
+    for (;;) {
+        uint64_t idle = __ballot(i < 0);
+        while (left && (int)__builtin_popcountll(idle) >= pathRefill(INST)) {
+            const int want = (int)__builtin_popcountll(idle), n = ctrv(cnt, part, kCQueue), start = partStart(cnt, part);
+            int b = 0;
+            if (laneId() == 0) b = atomicAdd(ctr(cnt, part, kCNext), want);
+            b = __builtin_amdgcn_readfirstlane(b);
+            if (i < 0) {
+                const int k = b + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
+                if (k < n) {
+                    i = start + k; depth = 0; T = v3(1.f, 1.f, 1.f); lastPdf = 0.f;
+                    cameraRay(F, i / K, (uint32_t)(smpBase + i % K), o, d);
+                }
+            }
+            if (b + want >= n) { left--; part = (part + 1) % kParts; }
+            idle = __ballot(i < 0);
+        }
+        if (idle == ~0ull) break;   // no path in this wave and none left
+        ShadeOut res;
+        res.cont = false; res.shadow = false; res.miss = false;
+        if (i >= 0) {
+            Hit h; h.t = 1e30f; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
+            traceRay<V, false, TRI, INST>(S, o, d, depth == 0 ? F.nearT : 0.f, h, st);
+            if constexpr (FULL) res = shadeFull<INST != 0>(S, P, F, depth, i, i / K, (uint32_t)(smpBase + i % K), o, d, T, lastPdf, h);
+            else res = shadeLegacy<INST != 0>(S, P, F, depth, i, i / K, (uint32_t)(smpBase + i % K), o, d, T, h);
+        }
+        bool vis = false;
+        if (res.shadow) {
+            Hit h; h.t = res.stmax; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
+            if (!traceRay<V, true, TRI, INST>(S, res.so, res.sdir, 0.f, h, st)) {
+                vis = true;
+                Vec4 l = P.L[i]; l.x += res.scon.x; l.y += res.scon.y; l.z += res.scon.z; P.L[i] = l;
+            }
+        }
+        nMiss += (int)__builtin_popcountll(__ballot(res.miss && depth > 0));
+        nMissCam += (int)__builtin_popcountll(__ballot(res.miss && depth == 0));
+        nShadow += (int)__builtin_popcountll(__ballot(res.shadow));
+        nUnocc += (int)__builtin_popcountll(__ballot(vis));
+        nCont += (int)__builtin_popcountll(__ballot(res.cont));
+        if (res.cont) { o = res.po; d = res.nd; T = res.Tn; lastPdf = res.pdf; depth++; }
+        else i = -1;
+    }
+    waveAdd(nMissCam, ctr(cnt, own, kCMiss));
+    waveAdd(nMiss, ctr(cnt + kCntStride, own, kCMiss));
+    waveAdd(nShadow, ctr(cnt, own, kCShadow));
+    waveAdd(nUnocc, ctr(cnt, own, kCUnocc));
+    waveAdd(nCont, ctr(cnt + kCntStride, own, kCQueue));
+}
+
 // Closest or any hit of explicit rays (parity and kernel-level entry point); two-level scenes also report the hit
 // instance (-1 on a miss) when hitInst is given.
 template <int V, int TRI, bool ANY, int SL, int INST>
@@ -1617,6 +1697,8 @@ struct Kernels {
     BounceFn bounceHandInst = nullptr, bounceHandFullInst = nullptr, bounceTailInst = nullptr, bounceTailFullInst = nullptr;
     BounceFn bounceTail2Inst = nullptr, bounceTail2FullInst = nullptr;
     ShadowFn shadowHandInst = nullptr, shadowTailInst = nullptr, shadowTail2Inst = nullptr;
+    // whole paths in one launch (one level; two levels with a BVH8 TLAS), legacy and full integrator
+    FirstFn path = nullptr, pathFull = nullptr, pathInst8 = nullptr, pathFullInst8 = nullptr;
     // depth 0 with the first-bounce sort fused in (kFirstTile-thread workgroups)
     FirstFn bounceFirst = nullptr, bounceFirstFull = nullptr;
     // the hand-off in batches (BVH8): pass kernels that hand off and their tails; rolling steps [full][per-lane]
@@ -1696,6 +1778,12 @@ void pickSL(int waves, Kernels& k) {
         k.bounceRollTail2[1][1] = k_bounce_roll_tail<TRI, SL, kFullWaves, true, true, 2>;
         k.shadowRollHand = k_shadow_roll<V, TRI, SL, true>;
         k.shadowRollTail = k_shadow_jobs_tail<TRI, SL, true, DevStepTable>;
+    }
+    k.path = k_path<V, TRI, SL, kOneLevel, false>;
+    k.pathFull = k_path<V, TRI, SL, kOneLevel, true>;
+    if constexpr (V == 8) {
+        k.pathInst8 = k_path<V, TRI, SL, kTlas8, false>;
+        k.pathFullInst8 = k_path<V, TRI, SL, kTlas8, true>;
     }
     k.bounceFirst = k_bounce_first<V, TRI, SL, 6, false>;
     k.bounceFirstFull = k_bounce_first<V, TRI, SL, kFullWaves, true>;

@@ -21,6 +21,15 @@ namespace cwp {
 enum LightMode { kLightMIS = 0, kLightNEE = 1, kLightBSDF = 2 };
 
 constexpr int kTailDefault = 12;   // hand-off threshold in lanes of the automatic setting (measured best of 6-16)
+// Most paths in flight for which a frame runs whole paths in one launch (k_path) instead of a queue per depth, where no
+// hand-off, sort, refill or register budget is asked for. Measured at 6 bounces, queues against k_path, ms per frame:
+// BVH8, terrain: 58 k paths 1.42 / 0.51, 0.9 M 2.14 / 1.35, 3.7 M 3.77 / 3.27, 5.5 M 4.84 / 4.60, 15 M 10.0 / 10.9 (queue
+// kernels hand stragglers off and trace compacted waves); full integrator 5.5 M 8.23 / 7.99, 15 M 18.4 / 20.1. BVH2: 15 M
+// 25.5 / 24.7, 59 M 95.0 / 96.1. BVH4: 59 M 75.0 / 69.4. Two levels: 0.2 M 8.8 / 3.8, 15 M 67.6 / 49.1, 59 M 236 / 187
+// (a wave's rays differ most there, and k_path gives idle lanes new paths).
+inline long long kPathMax(int variant, bool twoLevel) {
+    return twoLevel || variant == 4 ? 1ll << 31 : (variant == 2 ? 1ll << 24 : 6ll << 20);
+}
 struct RenderOptions {
     int variant = 8;        // BVH layout: 2 or 8 (compressed)
     int tri = kTriWoop;     // triangle test: kTriMT, kTriWoop, kTriWatertight

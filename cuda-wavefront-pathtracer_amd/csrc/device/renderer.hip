@@ -127,6 +127,8 @@ struct Renderer::Impl {
     BounceFn bounceTail2 = nullptr;                // second hand-off level (tailLevels 2)
     ShadowFn shadowTail2 = nullptr;
     int gridTail = 0, gridShadowTail = 0;
+    FirstFn path = nullptr;                        // whole paths in one launch (frames with few paths in flight)
+    int gridPath = 0;
     FirstFn bounceFirst = nullptr;                 // first-bounce sort fused into depth 0 (single-level scenes)
     int gridFirst = 0;                             // in kFirstTile-thread workgroups
     ShadowFn shadow = nullptr;
@@ -321,10 +323,14 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     }
     if (O.tail < -1 || O.tail == 1 || O.tail > kWave) { err = "tail must be -1 (auto), 0 (off) or 2..64 lanes"; return false; }
     if (O.tailLevels != 1 && O.tailLevels != 2) { err = "tail levels must be 1 or 2"; return false; }
+    const long long inFlight = (long long)F.cam.w * F.cam.h * std::max(O.batch, 1);
+    if (O.tail <= 0 && !O.sort && O.fuse && !O.persistent && !O.shadowRefill && O.bounceWaves == 8 &&
+        (!I.inst || I.tlasWide) && inFlight <= kPathMax(S.variant, I.inst))
+        I.path = I.inst ? (S.full ? I.kn.pathFullInst8 : I.kn.pathInst8) : (S.full ? I.kn.pathFull : I.kn.path);
     // two-level scenes hand off between node steps of either level, which needs the BVH8 TLAS
     const bool tailable = S.variant == 8 && (!I.inst || I.tlasWide) && O.fuse && !O.persistent;
-    // automatic: wherever it can run (single-level 720p frame 149.5 -> 138.6 ms, 1,001-instance frame 76.4 -> 74.1 ms)
-    I.O.tail = O.tail == -1 ? (tailable ? kTailDefault : 0) : O.tail;
+    // automatic: single-level scenes (720p frame 149.5 -> 138.6 ms); two-level ones run k_path
+    I.O.tail = O.tail == -1 ? (tailable && !I.inst && !I.path ? kTailDefault : 0) : O.tail;
     if (I.O.tail) {
         if (!tailable) {
             err = "the straggler hand-off (tail) needs a BVH8 scene (two-level: with the BVH8 TLAS) and the fused kernel "
@@ -368,10 +374,14 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     I.gridTail = I.bounceTail ? gridOf((const void*)I.bounceTail) : 0;
     if (I.bounceTail2) I.gridTail = std::min(I.gridTail, gridOf((const void*)I.bounceTail2));
     I.gridShadowTail = I.shadowTail ? gridOf((const void*)I.shadowTail) : 0;
+    if (I.path) {
+        const long long waves = (inFlight + kWave - 1) / kWave;
+        I.gridPath = (int)std::min<long long>(gridOf((const void*)I.path), (waves + kParts - 1) / kParts * kParts);
+    }
     I.maxGrid = std::max(std::max(std::max(I.gridBounce, I.gridTail), std::max(I.gridShadow, I.gridShadowTail)),
-                         std::max(I.gridTrace, I.gridFirst * (kFirstTile / kBlock)));
+                         std::max(std::max(I.gridTrace, I.gridPath), I.gridFirst * (kFirstTile / kBlock)));
     I.gridSort = std::max(kParts, 4 * numCU / kParts * kParts);
-    gridBlocks = I.gridBounce;
+    gridBlocks = I.path ? I.gridPath : I.gridBounce;
 
     // stack spill beyond the LDS part: the tree bounds the entries a traversal can hold (two-level scenes: the
     // deepest accepted TLAS below the deepest BLAS)
@@ -392,12 +402,13 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     I.NK = (int)NK;
     I.depths = O.bounces + 2;
     // ray sets by queue slot: depth d >= 1 reads set d & 1 and appends to the other (set 0 is read from depth 2 on,
-    // depth 1 reads set 1)
-    if (!I.alloc(I.P.O[0], NK, err) || !I.alloc(I.P.D[0], NK, err) || !I.alloc(I.P.T[0], NK, err) ||
-        !I.alloc(I.P.O[1], NK, err) || !I.alloc(I.P.D[1], NK, err) || !I.alloc(I.P.T[1], NK, err) ||
-        !I.alloc(I.P.L, NK, err) || !I.alloc(I.P.sO, NK, err) ||
-        !I.alloc(I.P.sD, NK, err) || !I.alloc(I.P.sC, NK, err) || !I.alloc(I.P.cnt, I.counterWords(), err) ||
-        !I.alloc(I.accum, (size_t)I.N, err) || !I.alloc(I.tot, kTot, err))
+    // depth 1 reads set 1); whole paths in one launch keep their rays in registers
+    if (!I.path && (!I.alloc(I.P.O[0], NK, err) || !I.alloc(I.P.D[0], NK, err) || !I.alloc(I.P.T[0], NK, err) ||
+                    !I.alloc(I.P.O[1], NK, err) || !I.alloc(I.P.D[1], NK, err) || !I.alloc(I.P.T[1], NK, err) ||
+                    !I.alloc(I.P.sO, NK, err) || !I.alloc(I.P.sD, NK, err) || !I.alloc(I.P.sC, NK, err)))
+        return false;
+    if (!I.alloc(I.P.L, NK, err) || !I.alloc(I.P.cnt, I.counterWords(), err) || !I.alloc(I.accum, (size_t)I.N, err) ||
+        !I.alloc(I.tot, kTot, err))
         return false;
     if (!O.fuse && !I.alloc(I.P.H, NK, err)) return false;
     if (O.sort < 0 || O.sort > 2) { err = "sort must be 0, 1 or 2"; return false; }
@@ -413,19 +424,9 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         const size_t records = ((NK >> 6) + kParts + 1) * (size_t)(I.O.tail - 1);
         // the second level's regions follow from the first's record numbering
         const size_t records2 = ((records >> 6) + kParts + 1) * (size_t)(I.O.tail - 1);
-        const bool ok = I.alloc(I.P.tail, records * (size_t)I.P.tailStride, err) &&
-                        (!I.bounceTail2 || I.alloc(I.P.tail2, records2 * (size_t)I.P.tailStride, err));
-        if (!ok) {
-            // the records of a two-level scene take up to 1.5 times the path state: where the automatic setting finds no
-            // room for them, the frame runs without the hand-off
-            if (!I.inst || O.tail != -1) return false;
-            (void)hipGetLastError();
-            if (I.P.tail) { hipFree(I.P.tail); I.allocs.pop_back(); }
-            I.P.tail = I.P.tail2 = nullptr; I.P.tailLanes = 0; I.O.tail = 0;
-            I.bounce = S.full ? I.kn.bounceFullInst8 : I.kn.bounceInst8; I.shadow = I.kn.shadowInst8;
-            I.bounceTail = I.bounceTail2 = nullptr; I.shadowTail = I.shadowTail2 = nullptr;
-            err.clear();
-        }
+        if (!I.alloc(I.P.tail, records * (size_t)I.P.tailStride, err) ||
+            (I.bounceTail2 && !I.alloc(I.P.tail2, records2 * (size_t)I.P.tailStride, err)))
+            return false;
     }
     HIPCHK(hipHostMalloc((void**)&I.hostTot, kTot * sizeof(unsigned long long), hipHostMallocDefault));
     int clockKHz = 0;
@@ -467,7 +468,11 @@ bool Renderer::render(int spp, int sBase, bool clear, FrameStats& S, std::string
             // first-bounce sort: the depth-0 launch stages its continuations, the later ones append directly
             DevPaths P0 = I.P, Pn = I.P;
             if (I.O.sort == 2) { P0.firstSort = I.bounceFirst ? 0 : 1; Pn.qk = nullptr; P0.qk = I.bounceFirst ? nullptr : P0.qk; }
-            for (int depth = 0; depth < I.depths; depth++) {
+            if (I.path) {
+                I.path<<<I.gridPath, kBlock, 0, I.st>>>(I.S, I.P, I.dF, s, I.K);
+                if (timed) S.bounceLaunches++;
+            }
+            for (int depth = 0; !I.path && depth < I.depths; depth++) {
                 if (depth == 0 && I.bounceFirst) {   // depth 0 with the first-bounce sort fused in
                     I.bounceFirst<<<I.gridFirst, kFirstTile, 0, I.st>>>(I.S, P0, I.dF, s, I.K);
                 } else {

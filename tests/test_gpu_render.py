@@ -390,3 +390,36 @@ def test_launch_times_and_totals_over_passes(extra, passes):
     np.testing.assert_array_equal(img, r.accum())
     for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
         assert st[key] == sum(s[key] for s in one), key
+
+
+PATH_SCENES = {"legacy": ["--gen", "terrain", "--gen_grid", "40", "--gen_boxes", "12"],
+               "full": ["--gen", "boxes", "--gen_boxes", "40", "--gen_materials", "3", "--gen_env", "64,32,1.5,2", "--rr", "1"],
+               "textured": ["--gen", "boxes", "--gen_boxes", "40", "--gen_materials", "3", "--gen_env", "64,32,1.5,2",
+                            "--gen_textures", "32"],
+               "two-level": ["--gen", "instances", "--gen_small", "1", "--gen_instances", "60"],
+               "two-level full": ["--gen", "instances", "--gen_small", "1", "--gen_instances", "60", "--gen_materials", "2",
+                                  "--gen_env", "64,32,1.5,2"]}
+
+
+@pytest.mark.parametrize("scene,variant,tri,size,extra", [
+    ("legacy", 8, "woop", (1, 1, 1), []), ("legacy", 8, "woop", (7, 1, 1), []), ("legacy", 8, "watertight", (97, 61, 3), []),
+    ("legacy", 8, "woop", (640, 360, 9), ["--aperture", "0.01", "--focus_dist", "0.8"]),   # more paths than resident lanes
+    ("legacy", 8, "woop", (65, 64, 2), ["--bounces", "0"]), ("legacy", 4, "mt", (65, 43, 5), []),
+    ("legacy", 2, "woop", (65, 43, 5), ["--stack", "32"]), ("full", 8, "woop", (65, 43, 4), []),
+    ("full", 2, "watertight", (64, 32, 3), []), ("textured", 8, "woop", (65, 43, 4), ["--graph", "0"]),
+    ("two-level", 8, "woop", (65, 43, 4), []), ("two-level", 8, "watertight", (320, 180, 12), []),
+    ("two-level full", 8, "woop", (65, 43, 4), [])])
+def test_whole_paths_equal_the_queue_kernels(scene, variant, tri, size, extra):
+    """Frames with few paths in flight run whole paths in one launch: image and ray counts are those of the queue kernels
+    (which any hand-off, sort, refill or register budget asks for), bit for bit, over one and several passes."""
+    print("case", scene, variant, tri, size, extra, flush=True)
+    w, h, k = size
+    args = PATH_SCENES[scene] + ["--variant", "bvh%d" % variant, "--tri", tri, "--width", str(w), "--height", str(h),
+                                 "--batch", str(k), "--bounces", "4"] + extra
+    one = cwp.Renderer(cwp.Setup(args))
+    queues = cwp.Renderer(cwp.Setup(args + (["--tail", "12"] if variant == 8 else ["--bounce_waves", "6"])))
+    for clear, base, passes in ((True, 0, 1), (False, k, 2)):
+        a, b = one.render(k * passes, base, clear), queues.render(k * passes, base, clear)
+        np.testing.assert_array_equal(one.accum(), queues.accum())
+        for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
+            assert a[key] == b[key], key
