@@ -40,7 +40,7 @@ constexpr int kParts = 8;        // queue partitions, one per XCD (workgroup w r
 // Line x: [kCQueue] path-queue length of partition x, [kCShadow] shadow rays it produced, [kCMiss] its misses,
 // [kCUnocc] its unoccluded shadow rays. Misses and unoccluded rays are summed per wave and added once at kernel end.
 constexpr int kLine = 32;
-constexpr int kCntStride = kParts * kLine;
+constexpr int kCntStride = 2 * kParts * kLine;   // the second half: hand-out counters (kW...), one line per partition
 constexpr int kCQueue = 0, kCShadow = 1, kCMiss = 2, kCUnocc = 3;
 // rolling batches (steps instead of passes) also keep per partition and step: [kCIn] rays the step traces (the previous
 // step's continuations + the step's camera rays), [kCMissCam] camera-ray misses
@@ -49,8 +49,9 @@ constexpr int kCIn = 4, kCMissCam = 5;
 constexpr int kCTail = 6, kCShadowTail = 7;   // ... and [kCShadowTail] the shadow kernel's
 // [kCTail2] / [kCShadowTail2]: traversals the first tail kernels handed on to the second ones
 constexpr int kCTail2 = 8, kCShadowTail2 = 9;
-// [kCNext] whole-path kernel: paths of the partition handed out
-constexpr int kCNext = 10;
+// Hand-out counters of a depth's launches, in the second half of its block: [kWPath] whole-path kernel: paths handed
+// out; the others: chunks of 64 entries handed out beyond those the waves take by themselves (Chunks)
+constexpr int kWPath = 0, kWBounce = 1, kWTail = 2, kWTail2 = 3, kWShadow = 4, kWShadowTail = 5, kWShadowTail2 = 6;
 // Device-clock stamps (64 bits each) in partition 0's line: when the depth's first trace+shade, tail, shade, shadow,
 // shadow-tail and sort launch began (0: no such launch). A launch's time is the next stamp minus its own (k_pass_end).
 // An event record between two launches costs 6-10 us of idle GPU, four of them per depth 0.32 ms of a ten-depth frame.
@@ -442,12 +443,67 @@ __device__ __forceinline__ void waveAdd(int count, int* counter) {
 __device__ __forceinline__ int* ctr(int* cnt, int part, int which) { return cnt + part * kLine + which; }
 __device__ __forceinline__ int ctrv(const int* cnt, int part, int which) { return cnt[part * kLine + which]; }
 
+// hand-out counter `which` of partition `part`
+__device__ __forceinline__ int* workCtr(int* cnt, int part, int which) { return cnt + (kParts + part) * kLine + which; }
+
 // start of partition `part` in a region laid out as the partitions' counts `which` of a counter block (default: the
 // queue lengths of a depth)
 __device__ __forceinline__ int partStart(const int* cnt, int part, int which = kCQueue) {
     int s = 0;
     for (int y = 0; y < part; y++) s += ctrv(cnt, y, which);
     return s;
+}
+
+// The 64-entry chunks of a launch, handed to its waves. A wave's first chunk is its own (chunk lw of its partition); the
+// rest of a partition is handed out by a counter, to its own waves and, once those find none left, to waves of the other
+// partitions: each tries one other partition (spread over all by lw) and stays with it. So neither a wave nor an XCD
+// idles while chunks are left, and a partition with at most a chunk per wave costs no atomics. Which wave traces a ray
+// changes nothing in its result; appends and tail records go to the chunk's partition.
+// Measured against every wave taking every nw-th chunk of its partition (720p terrain): 256 samples 144.2 -> 130.4 ms per
+// frame, 16 samples 11.5 -> 10.6, full integrator 64 samples 75.9 -> 65.1: bands of the image differ in the work per
+// ray. Half of the rounds fixed, the rest handed out: 131.2; three quarters fixed: 140.0. Trying two other partitions
+// instead of one: 11.2 -> 11.8 ms at 16 samples (failing atomics at the end of every launch), none: no gain at 256.
+struct Chunks {
+    int* next;        // the partitions' counters (workCtr of partition 0), kLine apart
+    int part, n;      // the partition chunks are taken from, its entries
+    int base;         // the current chunk's first entry
+    int lw, nw;
+    bool begun;       // the wave has had its own first chunk
+};
+__device__ __forceinline__ Chunks beginChunks(int* cnt, int which, int part, int n) {
+    Chunks c;
+    c.next = workCtr(cnt, 0, which);
+    c.part = part; c.n = n; c.base = 0; c.begun = false;
+    c.lw = (int)(blockIdx.x / kParts); c.nw = (int)(gridDim.x / kParts);
+    return c;
+}
+// the next chunk the counter of partition c.part hands out; false when it has none left
+__device__ __forceinline__ bool handChunk(Chunks& c) {
+    const int handed = ((c.n + kWave - 1) >> 6) - c.nw;   // chunks beyond the waves' own
+    if (handed <= 0) return false;
+    int b = 0;
+    if (laneId() == 0) b = atomicAdd(c.next + c.part * kLine, 1);
+    b = __builtin_amdgcn_readfirstlane(b);
+    c.base = (c.nw + b) * kWave;
+    return b < handed;
+}
+// The next chunk; false when none is left. moved: it is the first one from another partition (c.part). count(x): entries
+// of partition x.
+template <class Count>
+__device__ __forceinline__ bool nextChunk(Chunks& c, bool& moved, Count&& count) {
+    moved = false;
+    if (!c.begun) {
+        c.begun = true;
+        c.base = c.lw * kWave;
+        if (c.base < c.n) return true;
+    }
+    if (handChunk(c)) return true;
+    const int own = (int)(blockIdx.x % kParts);
+    if (c.part != own) return false;
+    c.part = (own + 1 + c.lw % (kParts - 1)) % kParts;
+    c.n = count(c.part);
+    moved = true;
+    return handChunk(c);
 }
 
 // camera ray of path (pix, smp): filter importance sampling (Blackman-Harris table or 1 px box), pinhole or thin lens
@@ -711,19 +767,21 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce(DevScene S, DevPaths P
     const int lane = laneId();
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
     stamp(cnt, kCStampBounce);
-    const int n = ctrv(cnt, part, kCQueue);
-    const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
-    const int outStart = partStart(cnt, part);
+    const int* inCnt = depth == 0 ? cnt : cnt - kCntStride;   // the input's partitions start at this block's prefix
+    Chunks c = beginChunks(cnt, kWBounce, own, ctrv(cnt, own, kCQueue));
+    int inStart = partStart(inCnt, own), outStart = partStart(cnt, own);
     int misses = 0;
-    for (int base = lw * kWave; base < n; base += nw * kWave) {
-        const int k = base + lane;
+    bool moved;
+    while (nextChunk(c, moved, [&](int x) { return ctrv(cnt, x, kCQueue); })) {
+        const int part = c.part, k = c.base + lane;
+        if (moved) { inStart = partStart(inCnt, part); outStart = partStart(cnt, part); }
         int i = 0;
         ShadeOut res;
         res.cont = false; res.shadow = false; res.miss = false;
-        if (k < n) {
+        if (k < c.n) {
             const int slot = inStart + k;
             Vec3 o, d; float tmin;
             pathRay(P, F, depth, slot, smpBase, K, i, o, d, tmin);
@@ -739,7 +797,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce(DevScene S, DevPaths P
         }
         misses += appendResults(P, cnt, part, outStart, depth, i, res);
     }
-    waveAdd(misses, ctr(cnt, part, kCMiss));
+    waveAdd(misses, ctr(cnt, own, kCMiss));
 }
 
 // Depth 0 with the first-bounce sort fused in: workgroups of kFirstTile threads (four waves, each with its own LDS
@@ -757,15 +815,34 @@ __global__ void __launch_bounds__(kFirstTile, WAVES) k_bounce_first(DevScene S, 
     const int gtid = blockIdx.x * kFirstTile + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + (threadIdx.x / kWave) * (SL > 0 ? SL : 1) * kWave + lane),
                          (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lb = (int)(blockIdx.x / kParts), nb = (int)(gridDim.x / kParts);
+    __shared__ int handed;
+    const int own = (int)(blockIdx.x % kParts), lb = (int)(blockIdx.x / kParts), nb = (int)(gridDim.x / kParts);
     int* cnt = P.cnt;
     stamp(cnt, kCStampBounce);
-    const int n = ctrv(cnt, part, kCQueue);
-    const int start = partStart(cnt, part);   // the depth-0 slots and the depth-1 queue of partition x start here
-    int* queue = ctr(cnt + kCntStride, part, kCQueue);
     int misses = 0;
-    for (int t0 = lb * kFirstTile; t0 < n; t0 += nb * kFirstTile) {   // block-uniform bound: every thread meets the barriers
-        const int k = t0 + (int)threadIdx.x;
+    // tiles as Chunks hands out chunks: a first one of its own, then by the partitions' counters, its own partition's
+    // first (block-uniform: every thread meets the barriers)
+    int part = own, left = kParts;
+    bool begun = false;
+    for (;;) {
+        const int n = ctrv(cnt, part, kCQueue), tiles = (n + kFirstTile - 1) / kFirstTile;
+        int tile = lb;
+        if (begun) {
+            if (threadIdx.x == 0) handed = nb < tiles ? atomicAdd(workCtr(cnt, part, kWBounce), 1) : tiles;
+            __syncthreads();
+            tile = nb + handed;
+            __syncthreads();
+        }
+        begun = true;
+        if (tile >= tiles) {
+            if (part == own && tile < nb) continue;   // no first tile: ask the counter
+            if (--left == 0) break;
+            part = (part + 1) % kParts;
+            continue;
+        }
+        const int start = partStart(cnt, part);   // the depth-0 slots and the depth-1 queue of partition x start here
+        int* queue = ctr(cnt + kCntStride, part, kCQueue);
+        const int k = tile * kFirstTile + (int)threadIdx.x;
         int i = 0;
         ShadeOut res;
         res.cont = false; res.shadow = false; res.miss = false;
@@ -786,7 +863,7 @@ __global__ void __launch_bounds__(kFirstTile, WAVES) k_bounce_first(DevScene S, 
             P.T[1][start + to] = v4(res.Tn, asFloat(1));
         }
     }
-    waveAdd(misses, ctr(cnt, part, kCMiss));
+    waveAdd(misses, ctr(cnt, own, kCMiss));
 }
 
 // The tails of a hand-off bounce, run after k_bounce<..., TAIL> of the same depth and before that depth's shadow
@@ -801,21 +878,23 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_tail(DevScene S, DevPa
     const int lane = laneId();
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<Group, SL> st{ (LdsPtr<Group>)(lds + threadIdx.x), (Group*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
     if (LEVEL == 1) stamp(cnt, kCStampTail);
-    const int nt = ctrv(cnt, part, LEVEL == 1 ? kCTail : kCTail2);
-    const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
-    const int outStart = partStart(cnt, part);
-    const size_t first1 = tailFirst(inStart, part, P.tailLanes), first2 = tailFirst(first1, part, P.tailLanes);
-    const Vec4* tail = LEVEL == 1 ? P.tail + first1 * (size_t)P.tailStride : P.tail2 + first2 * (size_t)P.tailStride;
+    const int* inCnt = depth == 0 ? cnt : cnt - kCntStride;
+    constexpr int kCount = LEVEL == 1 ? kCTail : kCTail2;
+    Chunks c = beginChunks(cnt, LEVEL == 1 ? kWTail : kWTail2, own, ctrv(cnt, own, kCount));
+    bool moved;
     int misses = 0;
-    for (int base = lw * kWave; base < nt; base += nw * kWave) {
-        const int k = base + lane;
+    while (nextChunk(c, moved, [&](int x) { return ctrv(cnt, x, kCount); })) {
+        const int part = c.part, k = c.base + lane;
+        const int inStart = partStart(inCnt, part), outStart = partStart(cnt, part);
+        const size_t first1 = tailFirst(inStart, part, P.tailLanes), first2 = tailFirst(first1, part, P.tailLanes);
+        const Vec4* tail = LEVEL == 1 ? P.tail + first1 * (size_t)P.tailStride : P.tail2 + first2 * (size_t)P.tailStride;
         int i = 0;
         ShadeOut res;
         res.cont = false; res.shadow = false; res.miss = false;
-        if (k < nt) {
+        if (k < c.n) {
             Hit h; TravState ts;
             const int slot = resumeRecord<INST>(tail + (size_t)k * P.tailStride, h, ts, st);
             Vec3 o, d; float tmin;
@@ -828,7 +907,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_tail(DevScene S, DevPa
         }
         misses += appendResults(P, cnt, part, outStart, depth, i, res);
     }
-    waveAdd(misses, ctr(cnt, part, kCMiss));
+    waveAdd(misses, ctr(cnt, own, kCMiss));
 }
 
 // Closest hits of the depth-`depth` queue with persistent lanes and dynamic ray fetching (after Aila & Laine 2009;
@@ -974,16 +1053,18 @@ __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow(DevSce
     __shared__ E lds[SL > 0 ? SL * kBlock : 1];
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
     stamp(cnt, kCStampShadow);
-    const int n = ctrv(cnt, part, kCShadow);
-    const int start = partStart(cnt, part);
+    Chunks c = beginChunks(cnt, kWShadow, own, ctrv(cnt, own, kCShadow));
+    int start = partStart(cnt, own);
+    bool moved;
     int unocc = 0;
-    for (int base = lw * kWave; base < n; base += nw * kWave) {
-        const int k = base + laneId();
+    while (nextChunk(c, moved, [&](int x) { return ctrv(cnt, x, kCShadow); })) {
+        const int part = c.part, k = c.base + laneId();
+        if (moved) start = partStart(cnt, part);
         bool vis = false;
-        if (k < n) {
+        if (k < c.n) {
             const Vec4 O = P.sO[start + k], D = P.sD[start + k];
             Hit h; h.t = D.w; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
             bool occluded;
@@ -997,13 +1078,13 @@ __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow(DevSce
             if (!occluded) {
                 vis = true;
                 const int i = asInt(O.w);
-                const Vec4 c = P.sC[start + k];
-                Vec4 l = P.L[i]; l.x += c.x; l.y += c.y; l.z += c.z; P.L[i] = l;
+                const Vec4 s = P.sC[start + k];
+                Vec4 l = P.L[i]; l.x += s.x; l.y += s.y; l.z += s.z; P.L[i] = l;
             }
         }
         unocc += (int)__builtin_popcountll(__ballot(vis));
     }
-    waveAdd(unocc, ctr(cnt, part, kCUnocc));
+    waveAdd(unocc, ctr(cnt, own, kCUnocc));
 }
 
 // The tails of a hand-off shadow kernel: its handed-off any-hit traversals resumed in full waves (LEVEL 1, handing
@@ -1013,18 +1094,20 @@ __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow_tail(D
     __shared__ Group lds[SL * kBlock];
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<Group, SL> st{ (LdsPtr<Group>)(lds + threadIdx.x), (Group*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
     if (LEVEL == 1) stamp(cnt, kCStampShadowTail);
-    const int nt = ctrv(cnt, part, LEVEL == 1 ? kCShadowTail : kCShadowTail2);
-    const int start = partStart(cnt, part);
-    const size_t first1 = tailFirst(start, part, P.tailLanes), first2 = tailFirst(first1, part, P.tailLanes);
-    const Vec4* tail = LEVEL == 1 ? P.tail + first1 * (size_t)P.tailStride : P.tail2 + first2 * (size_t)P.tailStride;
+    constexpr int kCount = LEVEL == 1 ? kCShadowTail : kCShadowTail2;
+    Chunks c = beginChunks(cnt, LEVEL == 1 ? kWShadowTail : kWShadowTail2, own, ctrv(cnt, own, kCount));
+    bool moved;
     int unocc = 0;
-    for (int base = lw * kWave; base < nt; base += nw * kWave) {
-        const int k = base + laneId();
+    while (nextChunk(c, moved, [&](int x) { return ctrv(cnt, x, kCount); })) {
+        const int part = c.part, k = c.base + laneId();
+        const int start = partStart(cnt, part);
+        const size_t first1 = tailFirst(start, part, P.tailLanes), first2 = tailFirst(first1, part, P.tailLanes);
+        const Vec4* tail = LEVEL == 1 ? P.tail + first1 * (size_t)P.tailStride : P.tail2 + first2 * (size_t)P.tailStride;
         bool vis = false;
-        if (k < nt) {
+        if (k < c.n) {
             Hit h; TravState ts;
             const int pos = resumeRecord<INST>(tail + (size_t)k * P.tailStride, h, ts, st);
             const Vec4 O = P.sO[pos], D = P.sD[pos];
@@ -1036,13 +1119,13 @@ __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_shadow_tail(D
             if (h.tri == -1) {
                 vis = true;
                 const int i = asInt(O.w);
-                const Vec4 c = P.sC[pos];
-                Vec4 l = P.L[i]; l.x += c.x; l.y += c.y; l.z += c.z; P.L[i] = l;
+                const Vec4 s = P.sC[pos];
+                Vec4 l = P.L[i]; l.x += s.x; l.y += s.y; l.z += s.z; P.L[i] = l;
             }
         }
         unocc += (int)__builtin_popcountll(__ballot(vis));
     }
-    waveAdd(unocc, ctr(cnt, part, kCUnocc));
+    waveAdd(unocc, ctr(cnt, own, kCUnocc));
 }
 
 // Shadow rays with persistent lanes and dynamic ray fetching (as k_trace_paths).
@@ -1137,7 +1220,7 @@ __global__ void __launch_bounds__(kBlock, FULL ? 4 : 5) k_path(DevScene S, DevPa
         while (left && (int)__builtin_popcountll(idle) >= pathRefill(INST)) {
             const int want = (int)__builtin_popcountll(idle), n = ctrv(cnt, part, kCQueue), start = partStart(cnt, part);
             int b = 0;
-            if (laneId() == 0) b = atomicAdd(ctr(cnt, part, kCNext), want);
+            if (laneId() == 0) b = atomicAdd(workCtr(cnt, part, kWPath), want);
             b = __builtin_amdgcn_readfirstlane(b);
             if (i < 0) {
                 const int k = b + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
@@ -1283,18 +1366,20 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_jobs(const DevJobTable
     const int lane = laneId();
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
-    const int n = ctrv(cnt, part, kCQueue);
-    const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
-    const int outStart = partStart(cnt, part);
+    const int* inCnt = depth == 0 ? cnt : cnt - kCntStride;
+    Chunks c = beginChunks(cnt, kWBounce, own, ctrv(cnt, own, kCQueue));
+    int inStart = partStart(inCnt, own), outStart = partStart(cnt, own);
+    bool moved;
     int misses = 0;
-    for (int b0 = lw * kWave; b0 < n; b0 += nw * kWave) {
-        const int k = b0 + lane;
+    while (nextChunk(c, moved, [&](int x) { return ctrv(cnt, x, kCQueue); })) {
+        const int part = c.part, k = c.base + lane;
+        if (moved) { inStart = partStart(inCnt, part); outStart = partStart(cnt, part); }
         int i = 0;
         ShadeOut res;
         res.cont = false; res.shadow = false; res.miss = false;
-        if (k < n) {
+        if (k < c.n) {
             const int slot = inStart + k;
             Vec3 o, d; float tmin;
             const JobEntry e = jobEntry(jobs, base, nJobs, P, depth, slot, o, d, tmin);
@@ -1310,7 +1395,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_jobs(const DevJobTable
         }
         misses += appendResults(P, cnt, part, outStart, depth, i, res);
     }
-    waveAdd(misses, ctr(cnt, part, kCMiss));
+    waveAdd(misses, ctr(cnt, own, kCMiss));
 }
 
 // The tail of a hand-off pass bounce (run after k_bounce_jobs<..., TAIL> of the same depth, before its shadow
@@ -1327,19 +1412,20 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_jobs_tail(const DevJob
     const int lane = laneId();
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<Group, SL> st{ (LdsPtr<Group>)(lds + threadIdx.x), (Group*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
-    const int nt = ctrv(cnt, part, kCTail);
-    const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
-    const int outStart = partStart(cnt, part);
-    const Vec4* tail = P.tail + tailFirst(inStart, part, P.tailLanes) * (size_t)P.tailStride;
+    const int* inCnt = depth == 0 ? cnt : cnt - kCntStride;
+    Chunks c = beginChunks(cnt, kWTail, own, ctrv(cnt, own, kCTail));
+    bool moved;
     int misses = 0;
-    for (int b0 = lw * kWave; b0 < nt; b0 += nw * kWave) {
-        const int k = b0 + lane;
+    while (nextChunk(c, moved, [&](int x) { return ctrv(cnt, x, kCTail); })) {
+        const int part = c.part, k = c.base + lane;
+        const int inStart = partStart(inCnt, part), outStart = partStart(cnt, part);
+        const Vec4* tail = P.tail + tailFirst(inStart, part, P.tailLanes) * (size_t)P.tailStride;
         int i = 0;
         ShadeOut res;
         res.cont = false; res.shadow = false; res.miss = false;
-        if (k < nt) {
+        if (k < c.n) {
             Hit h; TravState ts;
             const int slot = resumeRecord(tail + (size_t)k * P.tailStride, h, ts, st);
             Vec3 o, d; float tmin;
@@ -1352,7 +1438,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_jobs_tail(const DevJob
         }
         misses += appendResults(P, cnt, part, outStart, depth, i, res);
     }
-    waveAdd(misses, ctr(cnt, part, kCMiss));
+    waveAdd(misses, ctr(cnt, own, kCMiss));
 }
 
 // k_shadow over the shadow rays of many jobs: the ray's path id names its job and scene (TAIL: with the hand-off)
@@ -1367,15 +1453,17 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_jobs(const DevJobTable* __
     loadJobBases(jobs, nJobs, base);
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
-    const int n = ctrv(cnt, part, kCShadow);
-    const int start = partStart(cnt, part);
+    Chunks c = beginChunks(cnt, kWShadow, own, ctrv(cnt, own, kCShadow));
+    int start = partStart(cnt, own);
+    bool moved;
     int unocc = 0;
-    for (int b0 = lw * kWave; b0 < n; b0 += nw * kWave) {
-        const int k = b0 + laneId();
+    while (nextChunk(c, moved, [&](int x) { return ctrv(cnt, x, kCShadow); })) {
+        const int part = c.part, k = c.base + laneId();
+        if (moved) start = partStart(cnt, part);
         bool vis = false;
-        if (k < n) {
+        if (k < c.n) {
             const Vec4 O = P.sO[start + k], D = P.sD[start + k];
             const int i = asInt(O.w);
             const DevJob& J = jobs[jobOf(base, nJobs, i)];
@@ -1390,13 +1478,13 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_jobs(const DevJobTable* __
             }
             if (!occluded) {
                 vis = true;
-                const Vec4 c = P.sC[start + k];
-                Vec4 l = P.L[i]; l.x += c.x; l.y += c.y; l.z += c.z; P.L[i] = l;
+                const Vec4 s = P.sC[start + k];
+                Vec4 l = P.L[i]; l.x += s.x; l.y += s.y; l.z += s.z; P.L[i] = l;
             }
         }
         unocc += (int)__builtin_popcountll(__ballot(vis));
     }
-    waveAdd(unocc, ctr(cnt, part, kCUnocc));
+    waveAdd(unocc, ctr(cnt, own, kCUnocc));
 }
 
 // The tail of a hand-off batch shadow kernel: its handed-off any-hit traversals resumed to the end, each with the
@@ -1411,16 +1499,17 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_jobs_tail(const Table* __r
     loadJobBases(jobs, nJobs, base);
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<Group, SL> st{ (LdsPtr<Group>)(lds + threadIdx.x), (Group*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + (ROLL ? (x & 1) : x) * kCntStride;
-    const int nt = ctrv(cnt, part, kCShadowTail);
-    const int start = partStart(cnt, part, ROLL ? kCIn : kCQueue);
-    const Vec4* tail = P.tail + tailFirst(start, part, P.tailLanes) * (size_t)P.tailStride;
+    Chunks c = beginChunks(cnt, kWShadowTail, own, ctrv(cnt, own, kCShadowTail));
+    bool moved;
     int unocc = 0;
-    for (int b0 = lw * kWave; b0 < nt; b0 += nw * kWave) {
-        const int k = b0 + laneId();
+    while (nextChunk(c, moved, [&](int x) { return ctrv(cnt, x, kCShadowTail); })) {
+        const int part = c.part, k = c.base + laneId();
+        const int start = partStart(cnt, part, ROLL ? kCIn : kCQueue);
+        const Vec4* tail = P.tail + tailFirst(start, part, P.tailLanes) * (size_t)P.tailStride;
         bool vis = false;
-        if (k < nt) {
+        if (k < c.n) {
             Hit h; TravState ts;
             const int pos = resumeRecord(tail + (size_t)k * P.tailStride, h, ts, st);
             const Vec4 O = P.sO[pos], D = P.sD[pos];
@@ -1431,13 +1520,13 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_jobs_tail(const Table* __r
             while (!resumableStep<true, TRI, kOneLevel>(J.S, so, sd, 0.f, r, h, st, ts)) {}
             if (h.tri == -1) {
                 vis = true;
-                const Vec4 c = P.sC[pos];
-                Vec4 l = P.L[i]; l.x += c.x; l.y += c.y; l.z += c.z; P.L[i] = l;
+                const Vec4 s = P.sC[pos];
+                Vec4 l = P.L[i]; l.x += s.x; l.y += s.y; l.z += s.z; P.L[i] = l;
             }
         }
         unocc += (int)__builtin_popcountll(__ballot(vis));
     }
-    waveAdd(unocc, ctr(cnt, part, kCUnocc));
+    waveAdd(unocc, ctr(cnt, own, kCUnocc));
 }
 
 // ------------------------------------------------------------------------------------------------ rolling batches
@@ -1523,23 +1612,29 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_roll(const DevStepTabl
     const int lane = laneId();
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* blk = P.cnt + (step & 1) * kCntStride;
     const int* prev = P.cnt + ((step + 1) & 1) * kCntStride;
-    const int n = ctrv(blk, part, kCIn);
-    const int nCont = ctrv(prev, part, kCQueue);
-    const int contStart = partStart(prev, part, kCIn);
-    const int outStart = partStart(blk, part, kCIn);
-    const int camLo = (int)((long long)part * T->camPaths / kParts);
+    Chunks c = beginChunks(blk, kWBounce, own, ctrv(blk, own, kCIn));
+    int nCont, contStart, outStart, camLo;
+    auto enter = [&](int part) {
+        nCont = ctrv(prev, part, kCQueue);
+        contStart = partStart(prev, part, kCIn);
+        outStart = partStart(blk, part, kCIn);
+        camLo = (int)((long long)part * T->camPaths / kParts);
+    };
+    enter(own);
+    bool moved;
     const int inSet = step & 1, outSet = (step + 1) & 1;
     int misses = 0, camMisses = 0;
-    for (int b0 = lw * kWave; b0 < n; b0 += nw * kWave) {
-        const int k = b0 + lane;
+    while (nextChunk(c, moved, [&](int x) { return ctrv(blk, x, kCIn); })) {
+        const int part = c.part, k = c.base + lane;
+        if (moved) enter(part);
         int i = 0, depth = 0;
         bool cam = false;
         ShadeOut res;
         res.cont = false; res.shadow = false; res.miss = false;
-        if (k < n) {
+        if (k < c.n) {
             const int code = k < nCont ? contStart + k : -(camLo + (k - nCont)) - 1;
             cam = code < 0;
             Vec3 o, d; float tmin;
@@ -1557,8 +1652,8 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_roll(const DevStepTabl
         camMisses += (int)__builtin_popcountll(__ballot(cam && res.miss));
         misses += appendTo<LANE>(P, ctr(blk, part, kCQueue), ctr(blk, part, kCShadow), outStart, outSet, depth + 1, i, res);
     }
-    waveAdd(misses, ctr(blk, part, kCMiss));
-    waveAdd(camMisses, ctr(blk, part, kCMissCam));
+    waveAdd(misses, ctr(blk, own, kCMiss));
+    waveAdd(camMisses, ctr(blk, own, kCMissCam));
 }
 
 // The tails of a hand-off rolling step (after k_bounce_roll<..., TAIL>, before the step's shadow kernel), as those of a
@@ -1574,21 +1669,23 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_roll_tail(const DevSte
     const int lane = laneId();
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<Group, SL> st{ (LdsPtr<Group>)(lds + threadIdx.x), (Group*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* blk = P.cnt + (step & 1) * kCntStride;
-    const int nt = ctrv(blk, part, LEVEL == 1 ? kCTail : kCTail2);
-    const int outStart = partStart(blk, part, kCIn);
+    constexpr int kCount = LEVEL == 1 ? kCTail : kCTail2;
+    Chunks c = beginChunks(blk, LEVEL == 1 ? kWTail : kWTail2, own, ctrv(blk, own, kCount));
+    bool moved;
     const int inSet = step & 1, outSet = (step + 1) & 1;
-    const size_t first1 = tailFirst(outStart, part, P.tailLanes), first2 = tailFirst(first1, part, P.tailLanes);
-    const Vec4* tail = LEVEL == 1 ? P.tail + first1 * (size_t)P.tailStride : P.tail2 + first2 * (size_t)P.tailStride;
     int misses = 0, camMisses = 0;
-    for (int b0 = lw * kWave; b0 < nt; b0 += nw * kWave) {
-        const int k = b0 + lane;
+    while (nextChunk(c, moved, [&](int x) { return ctrv(blk, x, kCount); })) {
+        const int part = c.part, k = c.base + lane;
+        const int outStart = partStart(blk, part, kCIn);
+        const size_t first1 = tailFirst(outStart, part, P.tailLanes), first2 = tailFirst(first1, part, P.tailLanes);
+        const Vec4* tail = LEVEL == 1 ? P.tail + first1 * (size_t)P.tailStride : P.tail2 + first2 * (size_t)P.tailStride;
         int i = 0, depth = 0;
         bool cam = false;
         ShadeOut res;
         res.cont = false; res.shadow = false; res.miss = false;
-        if (k < nt) {
+        if (k < c.n) {
             Hit h; TravState ts;
             const int code = resumeRecord(tail + (size_t)k * P.tailStride, h, ts, st);
             cam = code < 0;
@@ -1605,8 +1702,8 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_roll_tail(const DevSte
         camMisses += (int)__builtin_popcountll(__ballot(cam && res.miss));
         misses += appendTo<LANE>(P, ctr(blk, part, kCQueue), ctr(blk, part, kCShadow), outStart, outSet, depth + 1, i, res);
     }
-    waveAdd(misses, ctr(blk, part, kCMiss));
-    waveAdd(camMisses, ctr(blk, part, kCMissCam));
+    waveAdd(misses, ctr(blk, own, kCMiss));
+    waveAdd(camMisses, ctr(blk, own, kCMissCam));
 }
 
 // the step's shadow rays (as k_shadow_jobs, counters of block step & 1; TAIL: with the hand-off)
@@ -1621,15 +1718,17 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_roll(const DevStepTable* _
     loadJobBases(jobs, nJobs, base);
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* blk = P.cnt + (step & 1) * kCntStride;
-    const int n = ctrv(blk, part, kCShadow);
-    const int start = partStart(blk, part, kCIn);
+    Chunks c = beginChunks(blk, kWShadow, own, ctrv(blk, own, kCShadow));
+    int start = partStart(blk, own, kCIn);
+    bool moved;
     int unocc = 0;
-    for (int b0 = lw * kWave; b0 < n; b0 += nw * kWave) {
-        const int k = b0 + laneId();
+    while (nextChunk(c, moved, [&](int x) { return ctrv(blk, x, kCShadow); })) {
+        const int part = c.part, k = c.base + laneId();
+        if (moved) start = partStart(blk, part, kCIn);
         bool vis = false;
-        if (k < n) {
+        if (k < c.n) {
             const Vec4 O = P.sO[start + k], D = P.sD[start + k];
             const int i = asInt(O.w);
             const DevJob& J = jobs[jobOf(base, nJobs, i)];
@@ -1644,13 +1743,13 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_roll(const DevStepTable* _
             }
             if (!occluded) {
                 vis = true;
-                const Vec4 c = P.sC[start + k];
-                Vec4 l = P.L[i]; l.x += c.x; l.y += c.y; l.z += c.z; P.L[i] = l;
+                const Vec4 s = P.sC[start + k];
+                Vec4 l = P.L[i]; l.x += s.x; l.y += s.y; l.z += s.z; P.L[i] = l;
             }
         }
         unocc += (int)__builtin_popcountll(__ballot(vis));
     }
-    waveAdd(unocc, ctr(blk, part, kCUnocc));
+    waveAdd(unocc, ctr(blk, own, kCUnocc));
 }
 
 // ------------------------------------------------------------------------------------------------------- dispatch

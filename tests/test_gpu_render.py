@@ -423,3 +423,20 @@ def test_whole_paths_equal_the_queue_kernels(scene, variant, tri, size, extra):
         np.testing.assert_array_equal(one.accum(), queues.accum())
         for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
             assert a[key] == b[key], key
+
+
+@pytest.mark.parametrize("extra", [["--tail", "12"], ["--tail", "2", "--tail_levels", "1"], ["--tail", "64", "--sort", "2"],
+                                   ["--variant", "bvh2", "--bounce_waves", "6"], ["--variant", "bvh4", "--bounce_waves", "6"],
+                                   ["--tail", "12", "--gen_materials", "3", "--gen_env", "64,32,1.5,2"]])
+def test_chunks_handed_out_equal_one_chunk_per_wave(extra):
+    """With one workgroup per CU most chunks of a launch are handed out by the partitions' counters, to other partitions'
+    waves too (the sky rows of this view leave some with little work); with the full grid every wave has at most its own.
+    Images and ray counts are equal, in a second frame too (the counters start anew)."""
+    print("case", extra, flush=True)
+    args = ["--gen", "boxes", "--gen_boxes", "200", "--width", "211", "--height", "157", "--batch", "8", "--bounces", "4"] + extra
+    few, many = (cwp.Renderer(cwp.Setup(args + ["--blocks_per_cu", n])) for n in ("1", "0"))
+    for base in (0, 8):
+        a, b = few.render(8, base), many.render(8, base)
+        np.testing.assert_array_equal(few.accum(), many.accum())
+        for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
+            assert a[key] == b[key], key

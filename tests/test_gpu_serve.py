@@ -376,3 +376,20 @@ def test_production_scale_scenes_alone_equal_mix_and_renderer():
     ref = r.accum()
     r.close()
     np.testing.assert_array_equal(mix[0], ref)
+
+
+@pytest.mark.parametrize("rolling,batched,full", [(1, True, 0), (0, True, 0), (1, False, 1), (1, True, 1)])
+def test_large_jobs_equal_the_renderer(rolling, batched, full):
+    """Jobs with more rays than a launch's lanes, whose chunks the partitions' counters hand out: a job of 2.6 M paths
+    beside smaller ones gives the single-job renderer's image bit for bit (same scene, size and samples in flight)."""
+    print("case", rolling, batched, full, flush=True)
+    args = BOXES + (["--gen_materials", "3", "--gen_env", "64,32,1.5,2"] if full else [])
+    w, h, spp = 401, 401, 16
+    srv = cwp.Server(variant=8, bounces=4, max_paths=1 << 24, rolling=rolling, full=full)
+    srv.add_scene(cwp.Setup(args + ["--bounces", "4"]))
+    imgs, infos, _ = run_jobs(srv, [(0, 40, 30, 4, 3, 5), (0, w, h, spp, 4, 7), (0, 64, 64, 2, 2, 4)], batched)
+    assert infos[1]["samples_per_pass"] == spp
+    r = cwp.Renderer(cwp.Setup(args + ["--width", str(w), "--height", str(h), "--batch", str(spp), "--bounces", "4",
+                                       "--tail", "12"]))
+    r.render(spp)
+    np.testing.assert_array_equal(imgs[1], r.accum())
