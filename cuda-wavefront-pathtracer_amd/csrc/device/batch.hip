@@ -227,7 +227,10 @@ bool BatchRenderer::init(const BatchOptions& O, std::string& err) {
     if (O.tail > 0 && O.variant != 8) { err = "batch: the straggler hand-off (tail) resumes BVH8 traversals only"; return false; }
     if (O.tailLevels != 1 && O.tailLevels != 2) { err = "batch: tail levels must be 1 or 2"; return false; }
     I.O = O; I.sl = O.stackLds;
-    I.O.tail = O.tail == -1 ? (O.variant == 8 ? kTailDefault : 0) : O.tail;
+    // automatic: off. Since waves take their chunks from counters the tail launches cost more than the lanes they free (64
+    // mixed jobs, rolling steps: 318 ms with 12 lanes and two levels, 307 without; one job at a time 517 / 483; 32 jobs of
+    // the full integrator 410 / 407, and 402 with one level).
+    I.O.tail = std::max(O.tail, 0);
     std::string name;
     if (!deviceInfo(I.numCU, name, err)) return false;
     HIPCHK(hipSetDevice(0));

@@ -22,14 +22,19 @@ enum LightMode { kLightMIS = 0, kLightNEE = 1, kLightBSDF = 2 };
 
 constexpr int kTailDefault = 12;   // hand-off threshold in lanes of the automatic setting (measured best of 6-16)
 // Most paths in flight for which a frame runs whole paths in one launch (k_path) instead of a queue per depth, where no
-// hand-off, sort, refill or register budget is asked for. Measured at 6 bounces, queues against k_path, ms per frame:
-// BVH8, terrain: 58 k paths 1.42 / 0.51, 0.9 M 2.14 / 1.35, 3.7 M 3.77 / 3.27, 5.5 M 4.84 / 4.60, 15 M 10.0 / 10.9 (queue
-// kernels hand stragglers off and trace compacted waves); full integrator 5.5 M 8.23 / 7.99, 15 M 18.4 / 20.1. BVH2: 15 M
-// 25.5 / 24.7, 59 M 95.0 / 96.1. BVH4: 59 M 75.0 / 69.4. Two levels: 0.2 M 8.8 / 3.8, 15 M 67.6 / 49.1, 59 M 236 / 187
-// (a wave's rays differ most there, and k_path gives idle lanes new paths).
-inline long long kPathMax(int variant, bool twoLevel) {
-    return twoLevel || variant == 4 ? 1ll << 31 : (variant == 2 ? 1ll << 24 : 6ll << 20);
+// hand-off, sort, refill or register budget is asked for. Measured at 1280x720, 6 bounces, queues against k_path, ms per
+// frame (1.84 M paths and so on for 2, 3, 4, 6 samples): BVH8 terrain 1.91 / 1.76, 2.37 / 2.37, 2.85 / 3.00, 3.72 / 4.16;
+// boxes 1.88 / 1.90; full integrator 1 sample 1.97 / 1.80, 2 samples 2.85 / 3.01. BVH2 4: 7.44 / 7.04, 6: 9.89 / 9.97, full
+// 2: 6.78 / 6.52, 3: 8.86 / 9.06. BVH4 4: 5.49 / 4.96, 6: 7.30 / 7.04. Two levels 4: 15.5 / 14.8, 6: 20.4 / 20.6, full 3:
+// 15.0 / 14.9, 4: 18.1 / 18.6. 58 k paths: 1.42 / 0.51 (BVH8), 5.6 / 3.8 (two levels, 0.2 M).
+inline long long kPathMax(int variant, bool twoLevel, bool full) {
+    return (variant == 8 && !twoLevel ? 1ll << 21 : 1ll << 22) >> (full ? 1 : 0);
 }
+// Fewest paths in flight for which the automatic setting hands stragglers off (to one tail launch). 720p terrain, 6
+// bounces, without / with, ms per frame: 16 samples 8.35 / 8.87, 32 15.69 / 15.72, 48 23.09 / 22.71, 64 30.4 / 29.5; full
+// integrator 16 15.6 / 15.9, 32 30.0 / 29.6; 256 samples, 8 bounces 128.5 / 123.8 (a second tail launch: 125.5). The tail
+// launches wait for single long rays; with few rays per depth that latency is more than the lanes they free.
+constexpr long long kTailMin = 1ll << 25;
 struct RenderOptions {
     int variant = 8;        // BVH layout: 2 or 8 (compressed)
     int tri = kTriWoop;     // triangle test: kTriMT, kTriWoop, kTriWatertight
@@ -50,7 +55,7 @@ struct RenderOptions {
                             // their own stragglers on to a second tail kernel)
     int tail = -1;          // straggler hand-off (BVH8, fused kernel): a trace+shade or shadow wave hands
                             // its tracing lanes to a tail kernel once fewer than this many remain (0: off; 2..64;
-                            // -1: kTailDefault where supported, else off)
+                            // -1: kTailDefault lanes and one level where supported and worth it (kTailMin), else off)
 };
 
 struct FrameStats {

@@ -325,12 +325,13 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     if (O.tailLevels != 1 && O.tailLevels != 2) { err = "tail levels must be 1 or 2"; return false; }
     const long long inFlight = (long long)F.cam.w * F.cam.h * std::max(O.batch, 1);
     if (O.tail <= 0 && !O.sort && O.fuse && !O.persistent && !O.shadowRefill && O.bounceWaves == 8 &&
-        (!I.inst || I.tlasWide) && inFlight <= kPathMax(S.variant, I.inst))
+        (!I.inst || I.tlasWide) && inFlight <= kPathMax(S.variant, I.inst, S.full != 0))
         I.path = I.inst ? (S.full ? I.kn.pathFullInst8 : I.kn.pathInst8) : (S.full ? I.kn.pathFull : I.kn.path);
     // two-level scenes hand off between node steps of either level, which needs the BVH8 TLAS
     const bool tailable = S.variant == 8 && (!I.inst || I.tlasWide) && O.fuse && !O.persistent;
-    // automatic: single-level scenes (720p frame 149.5 -> 138.6 ms); two-level ones run k_path
-    I.O.tail = O.tail == -1 ? (tailable && !I.inst && !I.path ? kTailDefault : 0) : O.tail;
+    // automatic: single-level scenes with many paths in flight, one level
+    I.O.tail = O.tail == -1 ? (tailable && !I.inst && inFlight >= kTailMin ? kTailDefault : 0) : O.tail;
+    const bool second = O.tail != -1 && O.tailLevels == 2;
     if (I.O.tail) {
         if (!tailable) {
             err = "the straggler hand-off (tail) needs a BVH8 scene (two-level: with the BVH8 TLAS) and the fused kernel "
@@ -341,7 +342,7 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
             I.bounce = S.full ? I.kn.bounceHandFullInst : I.kn.bounceHandInst;
             I.bounceTail = S.full ? I.kn.bounceTailFullInst : I.kn.bounceTailInst;
             I.shadow = I.kn.shadowHandInst; I.shadowTail = I.kn.shadowTailInst;
-            if (O.tailLevels == 2) {
+            if (second) {
                 I.bounceTail2 = S.full ? I.kn.bounceTail2FullInst : I.kn.bounceTail2Inst;
                 I.shadowTail2 = I.kn.shadowTail2Inst;
             }
@@ -349,7 +350,7 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
             I.bounce = S.full ? I.kn.bounceHandFull : I.kn.bounceHand;
             I.bounceTail = S.full ? I.kn.bounceTailFull : I.kn.bounceTail;
             if (!O.shadowRefill) { I.shadow = I.kn.shadowHand; I.shadowTail = I.kn.shadowTail; }
-            if (O.tailLevels == 2) {
+            if (second) {
                 I.bounceTail2 = S.full ? I.kn.bounceTail2Full : I.kn.bounceTail2;
                 if (I.shadowTail) I.shadowTail2 = I.kn.shadowTail2;
             }

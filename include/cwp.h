@@ -392,10 +392,9 @@ typedef struct cwp_server_options {
     int tail_lanes;                    /* straggler hand-off (BVH8 only) of the trace+shade launches, and with the
                                           full integrator of the shadow launches: a wave whose lanes still tracing
                                           drop below this many hands their traversals to a tail launch that resumes
-                                          them in full waves (images unchanged); -1 automatic
-                                          (12 with BVH8, else off), 0 off, 2..64; cwp_server_get_options reports
-                                          the resolved value. The autotuner keeps it for BVH8 trials and turns it
-                                          off for the others. */
+                                          them in full waves (images unchanged); -1 automatic (off: measured
+                                          faster), 0 off, 2..64; cwp_server_get_options reports the resolved value.
+                                          The autotuner keeps it for BVH8 trials and turns it off for the others. */
     int tail_levels;                   /* 2 (default): the rolling steps' trace+shade tail launches hand their own
                                           stragglers on to a second tail launch; 1: they resume every record to the
                                           end (as the pass mode's always do: a second level made it slower) */
