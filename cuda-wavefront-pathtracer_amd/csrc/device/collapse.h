@@ -34,8 +34,8 @@ public:
     CwbvhCollapser& operator=(const CwbvhCollapser&) = delete;
 
     // hnodes: device H-PLOC nodes of n primitives; nodesOut: device, room for 5 float4 per node (at most n nodes);
-    // primOut: device, n ints. Runs on `stream` and synchronises with it after the checks and once per 8 wide-tree levels. numNodes: the
-    // wide nodes written; depth: wide-tree levels.
+    // primOut: device, n ints. Runs on `stream` and synchronises with it. numNodes: the wide nodes written; depth:
+    // wide-tree levels.
     bool run(const Vec4* hnodes, int n, Vec4* nodesOut, int* primOut, void* stream, int& numNodes, int& depth, std::string& err);
     // the root's cost as one wide root (after run): the collapse's SAH is this over the root box's area
     float rootCost() const { return rootCost_; }

@@ -360,8 +360,8 @@ int cwp_hploc_to_bvh2(const void* hnodes, int n, void* out, void* stream);
 /* Compressed BVH8 (80-byte nodes, CWP_ARR_NODES layout) from H-PLOC nodes of n primitives, on the device: the
  * collapse of cwp_bvh_from_hploc with variant 8 (one primitive per binary leaf, SAH-optimal 8-wide collapse, octant
  * slot order, quantised child boxes), bit-identical to it. hnodes, nodes (room for 20 floats per primitive) and prims
- * (n ints: the leaf primitive order, i.e. CWP_ARR_ORDER) are device pointers; the call synchronises with `stream`
- * once per level of the wide tree. Replaces treeFromHploc + CWBVH::build on the host (src/accel/bvh_tools.cpp:12-168,
+ * (n ints: the leaf primitive order, i.e. CWP_ARR_ORDER) are device pointers; the call synchronises with
+ * `stream`. Replaces treeFromHploc + CWBVH::build on the host (src/accel/bvh_tools.cpp:12-168,
  * src/app/scene_setup.cpp:76-83). */
 int cwp_cwbvh_from_hploc(const void* hnodes, int n, void* nodes, int* num_nodes, void* prims, int* depth, void* stream);
 /* Host convenience for the same: uploads, collapses (timed with events: gpu_ms), downloads. */

@@ -95,3 +95,23 @@ def test_collapse_matches_host_deep_chain(n):
     compare(lo, hi, g)
     _, _, depth, _ = cwp.cwbvh_from_hploc_gpu(g, n)
     assert depth > 8
+
+
+@pytest.mark.parametrize("n", [7, 500, 8192, 8193, 9000])
+def test_collapse_of_a_caterpillar_tree(n):
+    """A tree in which every internal node has one leaf child: hundreds of wide levels of one node each, in one workgroup
+    (up to 8,192 primitives) or over many batches of level launches."""
+    print("case caterpillar n=%d" % n, flush=True)
+    rng = np.random.default_rng(n)
+    lo = np.zeros((n, 3), np.float32)
+    lo[:, 0] = np.arange(n)
+    lo[:, 1:] = rng.random((n, 2))
+    hi = lo + np.float32(0.5)
+    h = np.zeros((2 * n - 1, 8), np.float32)
+    ids = h.view(np.int32)
+    h[:n, 0:3], h[:n, 4:7] = lo, hi
+    ids[:n, 3], ids[:n, 7] = np.arange(n), -1
+    h[n:, 0:3], h[n:, 4:7] = np.minimum.accumulate(lo, 0)[1:], np.maximum.accumulate(hi, 0)[1:]
+    ids[n:, 3] = np.concatenate([[0], np.arange(n, 2 * n - 2)])
+    ids[n:, 7] = np.arange(1, n)
+    compare(lo, hi, h)
