@@ -506,6 +506,45 @@ __device__ __forceinline__ bool nextChunk(Chunks& c, bool& moved, Count&& count)
     return handChunk(c);
 }
 
+// The same for waves that refill idle lanes: entries of the current chunk are taken a few at a time ([cur, end) are left),
+// and the next chunk is fetched when they run out. A wave's lanes share a partition, so it changes to another one only
+// when all its lanes are idle (moveOn).
+struct Supply {
+    Chunks c;
+    int cur, end;
+    bool more;   // the partition may have entries left
+};
+__device__ __forceinline__ void fetchSupply(Supply& u) {
+    Chunks& c = u.c;
+    if (!c.begun) { c.begun = true; c.base = c.lw * kWave; u.more = c.base < c.n || handChunk(c); }
+    else u.more = handChunk(c);
+    u.cur = c.base;
+    u.end = u.more ? min(c.base + kWave, c.n) : c.base;
+}
+__device__ __forceinline__ Supply beginSupply(int* cnt, int which, int part, int n) {
+    Supply u;
+    u.c = beginChunks(cnt, which, part, n);
+    fetchSupply(u);
+    return u;
+}
+// this lane's next entry (for the lanes in `idle`; -1: none left in the chunk)
+__device__ __forceinline__ int takeEntry(Supply& u, uint64_t idle) {
+    const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
+    const int k = u.cur + rank < u.end ? u.cur + rank : -1;
+    u.cur = min(u.cur + (int)__builtin_popcountll(idle), u.end);
+    return ((idle >> laneId()) & 1u) ? k : -1;
+}
+// all lanes idle and the partition used up: on to another partition, once; false: the wave is done
+template <class Count>
+__device__ __forceinline__ bool moveOn(Supply& u, Count&& count) {
+    const int own = (int)(blockIdx.x % kParts);
+    if (u.c.part != own) return false;
+    u.c.part = (own + 1 + u.c.lw % (kParts - 1)) % kParts;
+    u.c.n = count(u.c.part);
+    fetchSupply(u);
+    return u.more;
+}
+
 // camera ray of path (pix, smp): filter importance sampling (Blackman-Harris table or 1 px box), pinhole or thin lens
 // (reference: src/render/wavefront.cu:43-57)
 __device__ __forceinline__ void cameraRay(const FrameParams& F, int pix, uint32_t smp, Vec3& o, Vec3& d) {
@@ -966,6 +1005,10 @@ __global__ void __launch_bounds__(kBlock, 8) k_trace_paths(DevScene S, DevPaths 
 // results, and take new rays from the partition's queue, while the other lanes keep their traversal state. A wave
 // therefore does not idle until its longest ray is done, and shading still runs on many lanes at once. Each path's
 // arithmetic is the one of k_bounce (same image); only the order of the appends differs.
+// The default for BVH2 (legacy): its rays need many short node visits, whose counts differ most between a wave's lanes,
+// and its small node step leaves registers for the state that lives through the shading (6 waves per SIMD; 8 spill more,
+// 4 hide less). 720p terrain, 64 samples, 6 bounces: trace+shade 63.1 -> 44.5 ms, with the refilled shadow kernel (18.6 ->
+// 16.9) 81.9 -> 61.5 per frame. BVH4 (47.6 -> 51.3) and BVH8 (6.4 -> 8.7 at 16 samples) are slower with it.
 template <int V, int TRI, int SL, int WAVES, bool FULL, int REFILL>
 __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_refill(DevScene S, DevPaths P, const FrameParams* __restrict__ Fp,
                                                                  int depth, int smpBase, int K) {
@@ -974,40 +1017,37 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_refill(DevScene S, Dev
     __shared__ E lds[SL > 0 ? SL * kBlock : 1];
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
     stamp(cnt, kCStampBounce);
-    const int n = ctrv(cnt, part, kCQueue);
-    const int inStart = depth == 0 ? partStart(cnt, part) : partStart(cnt - kCntStride, part);
-    const int outStart = partStart(cnt, part);
+    const int* inCnt = depth == 0 ? cnt : cnt - kCntStride;
+    Supply u = beginSupply(cnt, kWBounce, own, ctrv(cnt, own, kCQueue));
+    int inStart = partStart(inCnt, own), outStart = partStart(cnt, own);
     int slot = -1;                    // queue slot of this lane's ray, -1 = idle
     int i = 0;                        // its path id
     bool tracing = false;
     RayPre r; Hit h; TravState ts;
-    uint32_t f = 0;                   // wave-uniform: entries of the wave's share handed out so far
-    bool more = fetchPos(0, lw, nw) < n;
     int misses = 0;
     for (;;) {
-        const uint64_t idle = __ballot(slot < 0);
-        if (more && idle) {
-            if (slot < 0) {
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
-                const int k = fetchPos(f + rank, lw, nw);
-                if (k < n) {
-                    slot = inStart + k;
-                    Vec3 o, d; float tmin;
-                    pathRay(P, F, depth, slot, smpBase, K, i, o, d, tmin);
-                    r = prepareRay<TRI>(o, d, tmin);
-                    h.t = 1e30f; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
-                    travBegin(ts, S.root);
-                    st.sp = 0;
-                    tracing = true;
-                }
+        for (uint64_t idle = __ballot(slot < 0); u.more && idle; idle = __ballot(slot < 0)) {
+            if (u.cur == u.end) { fetchSupply(u); continue; }
+            const int k = takeEntry(u, idle);
+            if (k >= 0) {
+                slot = inStart + k;
+                Vec3 o, d; float tmin;
+                pathRay(P, F, depth, slot, smpBase, K, i, o, d, tmin);
+                r = prepareRay<TRI>(o, d, tmin);
+                h.t = 1e30f; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
+                travBegin(ts, S.root);
+                st.sp = 0;
+                tracing = true;
             }
-            f += (uint32_t)__builtin_popcountll(idle);
-            more = fetchPos(f, lw, nw) < n;
         }
-        if (__ballot(slot >= 0) == 0) break;   // no ray in flight: with `more` false the wave's share is done
+        if (__ballot(slot >= 0) == 0) {   // no ray in flight: this partition's share is done
+            if (!moveOn(u, [&](int x) { return ctrv(cnt, x, kCQueue); })) break;
+            inStart = partStart(inCnt, u.c.part); outStart = partStart(cnt, u.c.part);
+            continue;
+        }
         for (;;) {
             if (tracing) {
                 bool done;
@@ -1017,7 +1057,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_refill(DevScene S, Dev
                 if (done) tracing = false;
             }
             const uint64_t tr = __ballot(tracing);
-            if (tr == 0 || (more && (int)__builtin_popcountll(__ballot(slot >= 0 && !tracing)) >= REFILL)) break;
+            if (tr == 0 || (u.more && (int)__builtin_popcountll(__ballot(slot >= 0 && !tracing)) >= REFILL)) break;
         }
         const bool sh = slot >= 0 && !tracing;
         ShadeOut res;
@@ -1031,10 +1071,10 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_refill(DevScene S, Dev
                 res = shadeLegacy<false>(S, P, F, depth, i, i / K, (uint32_t)(smpBase + i % K), r.o, r.d, T, h);
             }
         }
-        misses += appendResults(P, cnt, part, outStart, depth, sh ? i : 0, res);
+        misses += appendResults(P, cnt, u.c.part, outStart, depth, sh ? i : 0, res);
         if (sh) slot = -1;
     }
-    waveAdd(misses, ctr(cnt, part, kCMiss));
+    waveAdd(misses, ctr(cnt, own, kCMiss));
 }
 
 // Shadow rays of bounce `depth` (partition per XCD as in k_bounce): any hit; unoccluded contributions are added to
@@ -1135,35 +1175,32 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_refill(DevScene S, DevPath
     __shared__ E lds[SL > 0 ? SL * kBlock : 1];
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    const int part = (int)(blockIdx.x % kParts), lw = (int)(blockIdx.x / kParts), nw = (int)(gridDim.x / kParts);
+    const int own = (int)(blockIdx.x % kParts);
     int* cnt = P.cnt + depth * kCntStride;
     stamp(cnt, kCStampShadow);
-    const int n = ctrv(cnt, part, kCShadow);
-    const int start = partStart(cnt, part);
+    Supply u = beginSupply(cnt, kWShadow, own, ctrv(cnt, own, kCShadow));
+    int start = partStart(cnt, own);
     int k = -1;                       // shadow-queue entry of this lane's ray, -1 = idle
     RayPre r; Hit h; TravState ts;
-    uint32_t f = 0;
-    bool more = fetchPos(0, lw, nw) < n;
     int unocc = 0;
     for (;;) {
-        const uint64_t idle = __ballot(k < 0);
-        if (more && (int)__builtin_popcountll(idle) >= REFILL) {
-            if (k < 0) {
-                const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
-                const int kk = fetchPos(f + rank, lw, nw);
-                if (kk < n) {
-                    k = kk;
-                    const Vec4 O = P.sO[start + k], D = P.sD[start + k];
-                    r = prepareRay<TRI>(xyz(O), xyz(D), 0.f);
-                    h.t = D.w; h.u = 0.f; h.v = 0.f; h.tri = -1;
-                    travBegin(ts, S.root);
-                    st.sp = 0;
-                }
+        for (uint64_t idle = __ballot(k < 0); u.more && (int)__builtin_popcountll(idle) >= REFILL; idle = __ballot(k < 0)) {
+            if (u.cur == u.end) { fetchSupply(u); continue; }
+            const int kk = takeEntry(u, idle);
+            if (kk >= 0) {
+                k = kk;
+                const Vec4 O = P.sO[start + k], D = P.sD[start + k];
+                r = prepareRay<TRI>(xyz(O), xyz(D), 0.f);
+                h.t = D.w; h.u = 0.f; h.v = 0.f; h.tri = -1;
+                travBegin(ts, S.root);
+                st.sp = 0;
             }
-            f += (uint32_t)__builtin_popcountll(idle);
-            more = fetchPos(f, lw, nw) < n;
         }
-        if (__ballot(k >= 0) == 0) break;
+        if (__ballot(k >= 0) == 0) {
+            if (!moveOn(u, [&](int x) { return ctrv(cnt, x, kCShadow); })) break;
+            start = partStart(cnt, u.c.part);
+            continue;
+        }
         if (k >= 0) {
             bool done;
             if constexpr (V == 2) done = stepBVH2<true, TRI>(S.nodes, S.tri, r, h, st, ts);
@@ -1183,7 +1220,7 @@ __global__ void __launch_bounds__(kBlock, 8) k_shadow_refill(DevScene S, DevPath
     // one atomic per wave for the unoccluded count
     int sum = unocc;
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-    waveAdd(sum, ctr(cnt, part, kCUnocc));
+    waveAdd(sum, ctr(cnt, own, kCUnocc));
 }
 
 // Whole paths in one launch: each lane carries a path from its camera ray to its end, tracing, shading and testing the
@@ -1872,7 +1909,7 @@ void pickSL(int waves, Kernels& k) {
     k.shadowJobs = k_shadow_jobs<V, TRI, SL>;
     k.bounceFull = k_bounce<V, TRI, SL, kFullWaves, kOneLevel, true>;
     k.bounceFullInst = k_bounce<V, TRI, SL, kFullWaves, kTlas2, true>;
-    k.bounceRefill = waves >= 8 ? k_bounce_refill<V, TRI, SL, 8, false, kShadeBatch>
+    k.bounceRefill = waves >= 8 && V != 2 ? k_bounce_refill<V, TRI, SL, 8, false, kShadeBatch>
                                 : (waves >= 6 ? k_bounce_refill<V, TRI, SL, 6, false, kShadeBatch> : k_bounce_refill<V, TRI, SL, 4, false, kShadeBatch>);
     k.bounceRefillFull = k_bounce_refill<V, TRI, SL, kFullWaves, true, kShadeBatch>;
     k.bounceJobsFull = k_bounce_jobs<V, TRI, SL, kFullWaves, true>;

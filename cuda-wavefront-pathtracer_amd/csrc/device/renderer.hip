@@ -327,6 +327,12 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     if (O.tail <= 0 && !O.sort && O.fuse && !O.persistent && !O.shadowRefill && O.bounceWaves == 8 &&
         (!I.inst || I.tlasWide) && inFlight <= kPathMax(S.variant, I.inst, S.full != 0))
         I.path = I.inst ? (S.full ? I.kn.pathFullInst8 : I.kn.pathInst8) : (S.full ? I.kn.pathFull : I.kn.path);
+    // BVH2 queues with the default schedule refill their lanes (k_bounce_refill's comment); the full integrator's trace+shade
+    // kernel has no registers left for that (25.6 -> 30.4 ms at 16 samples), its shadow rays do (10.5 -> 6.9)
+    if (S.variant == 2 && !I.inst && O.fuse && !O.persistent && !O.sort && O.bounceWaves == 8) {
+        if (!S.full) I.bounce = I.kn.bounceRefill;
+        I.shadow = I.kn.shadowRefill;
+    }
     // two-level scenes hand off between node steps of either level, which needs the BVH8 TLAS
     const bool tailable = S.variant == 8 && (!I.inst || I.tlasWide) && O.fuse && !O.persistent;
     // automatic: single-level scenes with many paths in flight, one level

@@ -427,6 +427,8 @@ def test_whole_paths_equal_the_queue_kernels(scene, variant, tri, size, extra):
 
 @pytest.mark.parametrize("extra", [["--tail", "12"], ["--tail", "2", "--tail_levels", "1"], ["--tail", "64", "--sort", "2"],
                                    ["--variant", "bvh2", "--bounce_waves", "6"], ["--variant", "bvh4", "--bounce_waves", "6"],
+                                   ["--variant", "bvh2", "--persistent", "2", "--shadow_refill", "1"],
+                                   ["--tail", "0", "--persistent", "2", "--shadow_refill", "1"],
                                    ["--tail", "12", "--gen_materials", "3", "--gen_env", "64,32,1.5,2"]])
 def test_chunks_handed_out_equal_one_chunk_per_wave(extra):
     """With one workgroup per CU most chunks of a launch are handed out by the partitions' counters, to other partitions'
@@ -440,3 +442,17 @@ def test_chunks_handed_out_equal_one_chunk_per_wave(extra):
         np.testing.assert_array_equal(few.accum(), many.accum())
         for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
             assert a[key] == b[key], key
+
+
+@pytest.mark.parametrize("extra", [[], ["--gen_materials", "3", "--gen_env", "64,32,1.5,2"]])
+def test_bvh2_default_schedule_equals_plain_queues(extra):
+    """BVH2 frames with more paths than whole-path launches take refill their lanes by default; image and ray counts are
+    those of the plain queue kernels, which a register budget asks for."""
+    print("case", extra, flush=True)
+    args = ["--gen", "boxes", "--gen_boxes", "60", "--width", "1001", "--height", "701", "--batch", "6", "--bounces", "3",
+            "--variant", "bvh2"] + extra
+    a, b = (cwp.Renderer(cwp.Setup(args + o)) for o in ([], ["--bounce_waves", "6"]))
+    x, y = a.render(6), b.render(6)
+    np.testing.assert_array_equal(a.accum(), b.accum())
+    for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
+        assert x[key] == y[key], key
