@@ -854,31 +854,14 @@ __global__ void __launch_bounds__(kFirstTile, WAVES) k_bounce_first(DevScene S, 
     const int gtid = blockIdx.x * kFirstTile + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + (threadIdx.x / kWave) * (SL > 0 ? SL : 1) * kWave + lane),
                          (E*)P.spill + (size_t)gtid * P.spillCap, 0, 0 };
-    __shared__ int handed;
-    const int own = (int)(blockIdx.x % kParts), lb = (int)(blockIdx.x / kParts), nb = (int)(gridDim.x / kParts);
+    const int part = (int)(blockIdx.x % kParts), lb = (int)(blockIdx.x / kParts), nb = (int)(gridDim.x / kParts);
     int* cnt = P.cnt;
     stamp(cnt, kCStampBounce);
     int misses = 0;
-    // tiles as Chunks hands out chunks: a first one of its own, then by the partitions' counters, its own partition's
-    // first (block-uniform: every thread meets the barriers)
-    int part = own, left = kParts;
-    bool begun = false;
-    for (;;) {
-        const int n = ctrv(cnt, part, kCQueue), tiles = (n + kFirstTile - 1) / kFirstTile;
-        int tile = lb;
-        if (begun) {
-            if (threadIdx.x == 0) handed = nb < tiles ? atomicAdd(workCtr(cnt, part, kWBounce), 1) : tiles;
-            __syncthreads();
-            tile = nb + handed;
-            __syncthreads();
-        }
-        begun = true;
-        if (tile >= tiles) {
-            if (part == own && tile < nb) continue;   // no first tile: ask the counter
-            if (--left == 0) break;
-            part = (part + 1) % kParts;
-            continue;
-        }
+    // every nb-th tile of the partition: handed out by counters as the other kernels' chunks are, the workgroup's four waves
+    // wait for each other and the counter (30.3 ms at 256 samples, asked for one tile ahead as slow, against 20.3)
+    const int n = ctrv(cnt, part, kCQueue);
+    for (int tile = lb; tile * kFirstTile < n; tile += nb) {   // block-uniform bound: every thread meets the barriers
         const int start = partStart(cnt, part);   // the depth-0 slots and the depth-1 queue of partition x start here
         int* queue = ctr(cnt + kCntStride, part, kCQueue);
         const int k = tile * kFirstTile + (int)threadIdx.x;
@@ -902,7 +885,7 @@ __global__ void __launch_bounds__(kFirstTile, WAVES) k_bounce_first(DevScene S, 
             P.T[1][start + to] = v4(res.Tn, asFloat(1));
         }
     }
-    waveAdd(misses, ctr(cnt, own, kCMiss));
+    waveAdd(misses, ctr(cnt, part, kCMiss));
 }
 
 // The tails of a hand-off bounce, run after k_bounce<..., TAIL> of the same depth and before that depth's shadow
