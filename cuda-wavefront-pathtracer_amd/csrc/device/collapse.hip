@@ -392,7 +392,8 @@ float hostArea(Vec3 lo, Vec3 hi) {
     return 2.f * (d.x * d.y + d.y * d.z + d.z * d.x);
 }
 
-constexpr size_t kLevelPad = 64;   // level records past the deepest possible level: a batch of empty levels
+constexpr int kFirstLevels = 16;   // levels queued before the host looks at the counts
+constexpr size_t kLevelPad = 64;   // level records past the deepest possible level: the first levels of a small tree
 Scratch carve(void* mem, int n) {
     const size_t N = 2 * (size_t)n - 1, M = (size_t)n;
     char* p = (char*)mem;
@@ -445,32 +446,41 @@ bool CwbvhCollapser::run(const Vec4* hn, int n, Vec4* nodesOut, int* primOut, vo
     k_cb_check<<<gN, 256, 0, st>>>(hn, n, W);
     k_cb_check2<<<gN, 256, 0, st>>>(n, W);
     if (n > 1) k_cb_dp<<<(n + 255) / 256, 256, 0, st>>>(hn, n, W);
-    // All launches are queued for as many levels as such a tree is expected to have (an empty level costs 3 us), then one
-    // wait; a deeper tree runs further batches of levels and the numbering again.
+    // As many levels as an ordinary tree has (2.02 M primitives: 12; an empty level costs 3 us) are queued with the
+    // numbering behind them, so the host waits once before it knows the tree's end. A deeper tree's numbering kernels do
+    // nothing then: batches of level launches follow, each as long as all before it (at most 1,024), with a look at the counts
+    // after each, and the numbering is queued once more when the last level is known. So a tree of L levels takes 3 L
+    // launches (with the numbering behind every 16 levels they were L^2 / 16): chains of 9,000 / 20,000 primitives (1,286 /
+    // 2,857 levels) 407 / 1,918 -> 46 / 86 ms, of 400,000 1.6 s.
     const bool one = n <= kOneBlock;
     const int top = one ? kOneBlock : kTopLevels;
     auto grid = [&](int l, int perNode) {   // level l holds at most 8^l nodes
         const long long nodes = l < 8 ? std::min<long long>(1ll << (3 * l), n) : n;
         return (int)std::max<long long>(1, std::min<long long>((nodes * perNode + 255) / 256, 2048));
     };
-    k_cb_top_down<<<1, kTopBlock, 0, st>>>(hn, n, top, n, W);
-    int levels = one ? 0 : 16;   // levels launched; batches of kLevelPad / 4
-    for (int l = kTopLevels; l < levels; l++) k_cb_level<<<grid(l, 8), 256, 0, st>>>(hn, n, l, n, W);
+    int levels = one ? 0 : kFirstLevels;   // levels launched
     struct { int ctl[2]; } head = {};
     int lastNum = 0;
-    for (;;) {
+    auto number = [&]() {
         for (int l = levels - 1; l >= kTopLevels; l--) k_cb_totals<<<grid(l, 1), 256, 0, st>>>(l, levels, W);
         k_cb_top_up<<<1, kTopBlock, 0, st>>>(levels, W);
         for (int l = kTopLevels; l < levels; l++) k_cb_offsets<<<grid(l, 1), 256, 0, st>>>(l, levels, W);
         k_cb_emit<<<(n + 255) / 256, 256, 0, st>>>(hn, n, levels, W, nodesOut, primOut);
+    };
+    k_cb_top_down<<<1, kTopBlock, 0, st>>>(hn, n, top, n, W);
+    for (int l = kTopLevels; l < levels; l++) k_cb_level<<<grid(l, 8), 256, 0, st>>>(hn, n, l, n, W);
+    number();
+    for (bool again = false;; again = true) {
         CCHK(hipMemcpyAsync(&head, W.ctl, sizeof head, hipMemcpyDeviceToHost, st));
         if (!one) CCHK(hipMemcpyAsync(&lastNum, W.num + levels, 4, hipMemcpyDeviceToHost, st));
         CCHK(hipStreamSynchronize(st));
         if (head.ctl[0] & 7) { err = "CWBVH collapse: the H-PLOC nodes are not a tree over [0, n) (code " + std::to_string(head.ctl[0]) + ")"; return false; }
         if (head.ctl[0]) { err = "CWBVH collapse: more wide nodes than primitives (code " + std::to_string(head.ctl[0]) + ")"; return false; }
-        if (one || lastNum == 0) break;
+        if (one || lastNum == 0) { if (again) number(); break; }
         if (levels >= n) { err = "CWBVH collapse: wide tree deeper than its primitive count"; return false; }
-        for (int k = 0; k < (int)kLevelPad / 4; k++, levels++) k_cb_level<<<grid(levels, 8), 256, 0, st>>>(hn, n, levels, n, W);
+        // up to the last level such a tree can have, n - 1 (the level records reach kLevelPad beyond it)
+        for (int k = std::min(std::min(levels, 1024), n - levels); k > 0; k--, levels++)
+            k_cb_level<<<grid(levels, 8), 256, 0, st>>>(hn, n, levels, n, W);
     }
     // the non-empty levels (a prefix), their end
     const int run = std::max(levels, head.ctl[1]);

@@ -97,10 +97,11 @@ def test_collapse_matches_host_deep_chain(n):
     assert depth > 8
 
 
-@pytest.mark.parametrize("n", [7, 500, 8192, 8193, 9000])
+@pytest.mark.parametrize("n", [7, 500, 8192, 8193, 9000, 100000])
 def test_collapse_of_a_caterpillar_tree(n):
     """A tree in which every internal node has one leaf child: hundreds of wide levels of one node each, in one workgroup
-    (up to 8,192 primitives) or over many batches of level launches."""
+    (up to 8,192 primitives) or over many batches of level launches. Three launches per level: 100,000 primitives (14,000
+    levels) take some 0.2 s (bounded at 3 s; launches that grow with the square of the levels take a minute)."""
     print("case caterpillar n=%d" % n, flush=True)
     rng = np.random.default_rng(n)
     lo = np.zeros((n, 3), np.float32)
@@ -115,3 +116,4 @@ def test_collapse_of_a_caterpillar_tree(n):
     ids[n:, 3] = np.concatenate([[0], np.arange(n, 2 * n - 2)])
     ids[n:, 7] = np.arange(1, n)
     compare(lo, hi, h)
+    assert cwp.cwbvh_from_hploc_gpu(h, n)[3] < 3000.0
