@@ -1285,62 +1285,87 @@ __global__ void __launch_bounds__(kBlock, FULL ? 4 : 5) k_path(DevScene S, DevPa
 }
 
 // Closest or any hit of explicit rays (parity and kernel-level entry point); two-level scenes also report the hit
-// instance (-1 on a miss) when hitInst is given. A wave walks the 64-ray chunks w, w + nw, ...; its idle lanes take the
-// next rays together once kTraceRefill are idle, so the lanes of short rays do not wait for the longest (a ray's state is
-// its traversal alone here, which fits the registers; in the fused kernels it did not). With at most a ray per lane
-// nothing is refilled. 4.2 M incoherent rays on the 118 k-triangle terrain, closest and any hits: 1.78 -> 1.48 ms (8 idle
-// lanes 1.49, 32 1.53).
-constexpr int kTraceRefill = 16;
-template <int V, int TRI, bool ANY, int SL, int INST>
+// instance (-1 on a miss) when hitInst is given. Bound by the latency of dependent node fetches and by lanes that wait for
+// their wave's longest ray.
+// REFILL, for queries of more rays than the grid has lanes: a wave walks the 64-ray chunks w, w + nw, ...; its idle lanes take
+// the next rays together once kTraceRefill are idle (a ray's state is its traversal alone here, which fits the registers).
+// Not while its chunks hold like rays (at most kTraceUnlike signs of direction components differ from the commoner ones:
+// 0 to 32 of 192 for camera rays, about 57 for a surface's hemispheres): their lanes read the same nodes, which rays from
+// elsewhere in the query beside them do not. 4.2 M rays on the 118 k-triangle terrain, closest / any hits, a ray per lane and
+// round, always refilled, with this rule: random surface points 1.03 / 0.73, 0.74 / 0.64, 0.73 / 0.64 ms; scan order of a
+// camera 0.329 / 0.268, 0.380 / 0.293, 0.330 / 0.271 ms. (8 idle lanes for 16: as fast, 32: 3 % slower. One loop for like and
+// unlike chunks: camera 0.338 / 0.281 ms, its register moves.)
+// Otherwise a ray per lane and round: with at most a ray per lane nothing can be refilled (20 k rays 61 us, 64 with the
+// refilling loop). Two-level scenes with a BVH2 TLAS nest their BLAS traversals in its loop and cannot refill.
+constexpr int kTraceRefill = 16, kTraceUnlike = 40;
+template <int V, int TRI, bool ANY, int SL, int INST, bool REFILL>
 __global__ void __launch_bounds__(kBlock, INST ? kInstWaves : 8) k_trace(DevScene S, const Vec4* __restrict__ rays, int n, Vec4* __restrict__ hits,
                                                      int* __restrict__ hitInst, void* spill, int spillCap) {
+    static_assert(!REFILL || INST != kTlas2, "the nested BLAS traversals cannot be suspended");
     using E = typename StackEntry<V>::type;
     __shared__ E lds[SL > 0 ? SL * kBlock : 1];
     const int gtid = blockIdx.x * kBlock + threadIdx.x;
     LaneStack<E, SL> st{ (LdsPtr<E>)(lds + threadIdx.x), (E*)spill + (size_t)gtid * spillCap, 0, 0 };
-    if constexpr (INST == kTlas2) {   // its BLAS traversals run nested in the TLAS loop: one ray per lane and round
+    auto traceOne = [&](int k) {
+        const Vec4 O = rays[2 * (size_t)k], D = rays[2 * (size_t)k + 1];
+        Hit h; h.t = D.w; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
+        traceRay<V, ANY, TRI, INST>(S, xyz(O), xyz(D), O.w, h, st);
+        hits[k] = v4(h.t, h.u, h.v, asFloat(h.tri));
+        if (hitInst) hitInst[k] = h.tri >= 0 ? h.inst : -1;
+    };
+    if constexpr (!REFILL) {
         for (int k = gtid; k - (int)threadIdx.x < n; k += gridDim.x * kBlock) {
             if (k >= n) continue;
-            const Vec4 O = rays[2 * (size_t)k], D = rays[2 * (size_t)k + 1];
-            Hit h; h.t = D.w; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
-            traceRay<V, ANY, TRI, INST>(S, xyz(O), xyz(D), O.w, h, st);
-            hits[k] = v4(h.t, h.u, h.v, asFloat(h.tri));
-            if (hitInst) hitInst[k] = h.tri >= 0 ? h.inst : -1;
+            traceOne(k);
         }
     } else {
         const long long nw = gridDim.x, w = blockIdx.x;
-        long long k = -1;        // this lane's ray, -1 = idle
+        uint32_t f = 0;          // wave-uniform: rays of the wave's chunks handed out so far
+        // chunk by chunk while the rays are alike (and the last chunk in any case)
+        for (;; f += kWave) {
+            const long long base = (w + (long long)(f >> 6) * nw) * kWave, k = base + laneId();
+            if (base >= n) return;
+            if (base + nw * kWave < n) {   // not the last chunk: every lane has a ray
+                const Vec4 D = rays[2 * k + 1];
+                auto fewer = [&](float x) { const int p = (int)__builtin_popcountll(__ballot(x < 0.f)); return min(p, kWave - p); };
+                if (fewer(D.x) + fewer(D.y) + fewer(D.z) > kTraceUnlike) break;
+            }
+            if (k < n) traceOne((int)k);
+        }
+        int k = -1;              // this lane's ray, -1 = idle
+        // the stack once more, from the lane id: carried across both loops its spill address does not fit the registers
+        LaneStack<E, SL> sr{ (LdsPtr<E>)(lds + laneId()), (E*)spill + ((size_t)blockIdx.x * kBlock + laneId()) * spillCap, 0, 0 };
         Vec3 o, d;               // the world ray (two-level scenes)
         float tmin = 0.f;
         o = d = v3(0.f, 0.f, 0.f);
         RayPre r; Hit h; TravState ts;
-        uint32_t f = 0;          // wave-uniform: rays of the wave's chunks handed out so far
-        bool more = w * kWave < n;
+        bool more = true;
         for (;;) {
             const uint64_t idle = __ballot(k < 0);
-            if (more && (int)__builtin_popcountll(idle) >= kTraceRefill) {
+            if (more) {
                 if (k < 0) {
                     const uint32_t g = f + __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
                     const long long kk = (w + (long long)(g >> 6) * nw) * kWave + (g & 63u);
                     if (kk < n) {
-                        k = kk;
-                        const Vec4 O = rays[2 * k], D = rays[2 * k + 1];
+                        k = (int)kk;
+                        const Vec4 O = rays[2 * kk], D = rays[2 * kk + 1];
                         o = xyz(O); d = xyz(D); tmin = O.w;
                         r = prepareRay<TRI>(o, d, tmin);
                         h.t = D.w; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1;
                         travBegin(ts, INST ? 0 : S.root);
-                        st.sp = 0; st.floor = 0;
+                        sr.sp = 0; sr.floor = 0;
                     }
                 }
                 f += (uint32_t)__builtin_popcountll(idle);
                 more = (w + (long long)(f >> 6) * nw) * kWave + (f & 63u) < n;
-            }
-            if (__ballot(k >= 0) == 0) break;   // no ray in flight: with `more` false the wave's chunks are done
+            } else if (idle == ~0ull) return;
             if (k >= 0) {
                 bool done;
-                if constexpr (V == 2) done = stepBVH2<ANY, TRI>(S.nodes, S.tri, r, h, st, ts);
-                else if constexpr (V == 4) done = stepBVH4<ANY, TRI>(S.nodes, S.tri, r, h, st, ts);
-                else done = resumableStep<ANY, TRI, INST>(S, o, d, tmin, r, h, st, ts);
+                do {
+                    if constexpr (V == 2) done = stepBVH2<ANY, TRI>(S.nodes, S.tri, r, h, sr, ts);
+                    else if constexpr (V == 4) done = stepBVH4<ANY, TRI>(S.nodes, S.tri, r, h, sr, ts);
+                    else done = resumableStep<ANY, TRI, INST>(S, o, d, tmin, r, h, sr, ts);
+                } while (!done && (int)__builtin_popcountll(__ballot(true)) > (more ? kWave - kTraceRefill : 0));
                 if (done) {
                     hits[k] = v4(h.t, h.u, h.v, asFloat(h.tri));
                     if (hitInst) hitInst[k] = h.tri >= 0 ? h.inst : -1;
@@ -1836,15 +1861,15 @@ struct Kernels {
     BounceFn bounce = nullptr;                          // fused trace + shade
     BounceFn tracePaths = nullptr, tracePlain = nullptr; // split: closest-hit trace with / without refill (then k_shade)
     ShadowFn shadow = nullptr, shadowRefill = nullptr;
-    TraceFn traceC = nullptr, traceA = nullptr;
+    TraceFn trace[2] = {}, traceMany[2] = {};   // [any hit]; one ray per lane and round, lanes refilled
     // two-level scenes (fused bounce kernel only)
     BounceFn bounceInst = nullptr;
     ShadowFn shadowInst = nullptr;
-    TraceFn traceCInst = nullptr, traceAInst = nullptr;
+    TraceFn traceInst[2] = {};
     // the same with a BVH8 TLAS (BVH8 BLASes)
     BounceFn bounceInst8 = nullptr, bounceFullInst8 = nullptr;
     ShadowFn shadowInst8 = nullptr;
-    TraceFn traceCInst8 = nullptr, traceAInst8 = nullptr;
+    TraceFn traceInst8[2] = {}, traceManyInst8[2] = {};
     // batched jobs
     JobsFn bounceJobs = nullptr, shadowJobs = nullptr;
     // full material integrator (fused bounce kernel; shadow rays use the legacy shadow kernels)
@@ -1882,12 +1907,14 @@ void pickSL(int waves, Kernels& k) {
     k.tracePlain = k_trace_paths<V, TRI, SL, kWave>;
     k.shadow = k_shadow<V, TRI, SL, kOneLevel>;
     k.shadowRefill = k_shadow_refill<V, TRI, SL, kRefill>;
-    k.traceC = k_trace<V, TRI, false, SL, kOneLevel>;
-    k.traceA = k_trace<V, TRI, true, SL, kOneLevel>;
+    k.trace[0] = k_trace<V, TRI, false, SL, kOneLevel, false>;
+    k.trace[1] = k_trace<V, TRI, true, SL, kOneLevel, false>;
+    k.traceMany[0] = k_trace<V, TRI, false, SL, kOneLevel, true>;
+    k.traceMany[1] = k_trace<V, TRI, true, SL, kOneLevel, true>;
     k.bounceInst = k_bounce<V, TRI, SL, kInstWaves, kTlas2>;
     k.shadowInst = k_shadow<V, TRI, SL, kTlas2>;
-    k.traceCInst = k_trace<V, TRI, false, SL, kTlas2>;
-    k.traceAInst = k_trace<V, TRI, true, SL, kTlas2>;
+    k.traceInst[0] = k_trace<V, TRI, false, SL, kTlas2, false>;
+    k.traceInst[1] = k_trace<V, TRI, true, SL, kTlas2, false>;
     k.bounceJobs = k_bounce_jobs<V, TRI, SL, 8>;
     k.shadowJobs = k_shadow_jobs<V, TRI, SL>;
     k.bounceFull = k_bounce<V, TRI, SL, kFullWaves, kOneLevel, true>;
@@ -1920,8 +1947,10 @@ void pickSL(int waves, Kernels& k) {
         k.bounceInst8 = k_bounce<V, TRI, SL, kInstWaves, kTlas8>;
         k.bounceFullInst8 = k_bounce<V, TRI, SL, kFullWaves, kTlas8, true>;
         k.shadowInst8 = k_shadow<V, TRI, SL, kTlas8>;
-        k.traceCInst8 = k_trace<V, TRI, false, SL, kTlas8>;
-        k.traceAInst8 = k_trace<V, TRI, true, SL, kTlas8>;
+        k.traceInst8[0] = k_trace<V, TRI, false, SL, kTlas8, false>;
+        k.traceInst8[1] = k_trace<V, TRI, true, SL, kTlas8, false>;
+        k.traceManyInst8[0] = k_trace<V, TRI, false, SL, kTlas8, true>;
+        k.traceManyInst8[1] = k_trace<V, TRI, true, SL, kTlas8, true>;
         k.shadowHandInst = k_shadow<V, TRI, SL, kTlas8, true>;
         k.shadowTailInst = k_shadow_tail<TRI, SL, 1, kTlas8>;
         k.shadowTail2Inst = k_shadow_tail<TRI, SL, 2, kTlas8>;

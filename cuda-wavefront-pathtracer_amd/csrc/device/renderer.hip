@@ -132,7 +132,7 @@ struct Renderer::Impl {
     FirstFn bounceFirst = nullptr;                 // first-bounce sort fused into depth 0 (single-level scenes)
     int gridFirst = 0;                             // in kFirstTile-thread workgroups
     ShadowFn shadow = nullptr;
-    int gridBounce = 0, gridShade = 0, gridShadow = 0, gridTrace = 0, maxGrid = 0, gridSort = 0;
+    int gridBounce = 0, gridShade = 0, gridShadow = 0, gridTrace = 0, gridTraceMany = 0, maxGrid = 0, gridSort = 0;
     void* stageRays = nullptr; void* stageHits = nullptr; int* stageInst = nullptr; size_t stageCap = 0;   // traceHost staging
     // two-level scenes: instance records, their world boxes, the TLAS (H-PLOC each frame), BLAS roots per mesh
     bool inst = false, instSet = false;
@@ -309,10 +309,10 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         I.shade = nullptr;
         if (I.tlasWide) {
             I.bounce = S.full ? I.kn.bounceFullInst8 : I.kn.bounceInst8; I.shadow = I.kn.shadowInst8;
-            I.kn.traceC = I.kn.traceCInst8; I.kn.traceA = I.kn.traceAInst8;
+            for (int a = 0; a < 2; a++) { I.kn.trace[a] = I.kn.traceInst8[a]; I.kn.traceMany[a] = I.kn.traceManyInst8[a]; }
         } else {
             I.bounce = S.full ? I.kn.bounceFullInst : I.kn.bounceInst; I.shadow = I.kn.shadowInst;
-            I.kn.traceC = I.kn.traceCInst; I.kn.traceA = I.kn.traceAInst;
+            for (int a = 0; a < 2; a++) I.kn.trace[a] = I.kn.traceMany[a] = I.kn.traceInst[a];
         }
         HIPCHK(hipHostMalloc((void**)&I.hostDepth, 2 * sizeof(int), hipHostMallocDefault));   // TLAS depth, build status
         if (!I.alloc(I.dDepth, 1, err)) return false;
@@ -371,7 +371,8 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     I.gridBounce = gridOf((const void*)I.bounce);
     I.gridShade = I.shade ? gridOf((const void*)I.shade) : 0;
     I.gridShadow = gridOf((const void*)I.shadow);
-    I.gridTrace = std::max(gridOf((const void*)I.kn.traceC), gridOf((const void*)I.kn.traceA));
+    I.gridTrace = std::max(gridOf((const void*)I.kn.trace[0]), gridOf((const void*)I.kn.trace[1]));
+    I.gridTraceMany = std::max(gridOf((const void*)I.kn.traceMany[0]), gridOf((const void*)I.kn.traceMany[1]));
     if (O.sort == 2 && !I.inst && O.fuse && !O.persistent) {
         I.bounceFirst = S.full ? I.kn.bounceFirstFull : I.kn.bounceFirst;
         int b = 0;
@@ -386,7 +387,7 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         I.gridPath = (int)std::min<long long>(gridOf((const void*)I.path), (waves + kParts - 1) / kParts * kParts);
     }
     I.maxGrid = std::max(std::max(std::max(I.gridBounce, I.gridTail), std::max(I.gridShadow, I.gridShadowTail)),
-                         std::max(std::max(I.gridTrace, I.gridPath), I.gridFirst * (kFirstTile / kBlock)));
+                         std::max(std::max(std::max(I.gridTrace, I.gridTraceMany), I.gridPath), I.gridFirst * (kFirstTile / kBlock)));
     I.gridSort = std::max(kParts, 4 * numCU / kParts * kParts);
     gridBlocks = I.path ? I.gridPath : I.gridBounce;
 
@@ -564,8 +565,10 @@ bool Renderer::trace(const void* rays, int n, bool anyHit, void* hits, std::stri
     if (n < 0) { err = "negative ray count"; return false; }
     if (n == 0) return true;
     if (I.inst && !I.instSet) { err = "two-level scene: set the instances of a frame first"; return false; }
-    TraceFn fn = anyHit ? I.kn.traceA : I.kn.traceC;
-    fn<<<I.gridTrace, kBlock, 0, I.st>>>(I.S, (const Vec4*)rays, n, (Vec4*)hits, inst, I.P.spill, I.P.spillCap);
+    // more rays than lanes: idle lanes take the rest (k_trace)
+    const bool many = n > (long long)I.gridTrace * kBlock;
+    TraceFn fn = (many ? I.kn.traceMany : I.kn.trace)[anyHit ? 1 : 0];
+    fn<<<many ? I.gridTraceMany : I.gridTrace, kBlock, 0, I.st>>>(I.S, (const Vec4*)rays, n, (Vec4*)hits, inst, I.P.spill, I.P.spillCap);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(I.st));
     return true;

@@ -183,6 +183,36 @@ def test_overlapping_instances(tri, stack, tail, count):
     np.testing.assert_array_equal(r.accum(), plain.accum())
 
 
+@pytest.mark.parametrize("tri,tlas,n", [("woop", "bvh8", 16384), ("woop", "bvh8", 16385), ("watertight", "bvh8", 60001),
+                                        ("mt", "bvh8", 40000), ("woop", "bvh2", 40001)])
+def test_two_level_queries_of_more_rays_than_lanes(tri, tlas, n):
+    """With one workgroup per CU (16,384 lanes on 256 CUs) idle lanes take new rays beside lanes inside a BLAS (BVH8 TLAS;
+    a BVH2 TLAS goes round by round): hits and instance ids bit for bit those of the full grid, which has a lane for
+    every ray here, and the oracle's on all but grazing rays."""
+    print("case", tri, tlas, n, flush=True)
+    args = ARGS + ["--tri", tri, "--tlas", tlas]
+    s = cwp.Setup(args)
+    few, full = (cwp.Renderer(cwp.Setup(args + ["--blocks_per_cu", b])) for b in ("1", "0"))
+    few.set_frame(0)
+    full.set_frame(0)
+    rng = np.random.default_rng(n)
+    d = rng.normal(size=(n, 3))
+    d[:n // 3] = np.abs(d[:n // 3]) * [1, 1, -1]   # like rays first: the waves' first chunks are traced whole
+    rays = np.concatenate([rng.uniform([-12, -12, -1], [12, 12, 3], (n, 3)), np.zeros((n, 1)),
+                           d / np.linalg.norm(d, axis=1, keepdims=True),
+                           np.where(rng.random((n, 1)) < 0.3, rng.uniform(1, 10, (n, 1)), 1e30)], 1).astype(np.float32)
+    (g, gi), (f, fi) = few.trace_inst(rays), full.trace_inst(rays)
+    np.testing.assert_array_equal(g.view(np.uint32), f.view(np.uint32))
+    np.testing.assert_array_equal(gi, fi)
+    hit = g[:, 3].view(np.int32) >= 0
+    assert 0.2 < hit.mean() < 0.95 and np.array_equal(gi >= 0, hit)
+    a, ai = few.trace_inst(rays, any_hit=True)
+    np.testing.assert_array_equal(a[:, 3].view(np.int32) >= 0, hit)
+    np.testing.assert_array_equal(ai >= 0, hit)
+    o, oi = oracle_scene(s, 0, {"mt": 0, "woop": 1, "watertight": 2}[tri]).trace_inst(rays)
+    assert ((g[:, 3].view(np.int32) == o[:, 3].view(np.int32)) & (gi == oi)).mean() >= 0.999
+
+
 FULL = ARGS + ["--gen_materials", "2", "--gen_env", "64,32,1.5,2", "--bounces", "3"]
 
 

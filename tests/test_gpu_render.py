@@ -456,3 +456,36 @@ def test_bvh2_default_schedule_equals_plain_queues(extra):
     np.testing.assert_array_equal(a.accum(), b.accum())
     for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
         assert x[key] == y[key], key
+
+
+@pytest.mark.parametrize("variant,tri,n", [(8, "woop", 16384), (8, "woop", 16385), (8, "woop", 100003), (8, "watertight", 40001),
+                                           (4, "mt", 40001), (2, "woop", 70000)])
+def test_queries_of_more_rays_than_lanes(variant, tri, n):
+    """Ray queries of more rays than the grid has lanes (one workgroup per CU: 16,384 on 256 CUs) give their idle lanes new
+    rays in mid-traversal of the others; smaller ones trace a ray per lane. Hits are bit for bit those of the full grid,
+    which has a lane for every ray here, and match the oracle's, with ranges that end some rays early."""
+    print("case", variant, tri, n, flush=True)
+    args = ["--gen", "terrain", "--gen_grid", "80", "--width", "16", "--height", "16", "--variant", "bvh%d" % variant, "--tri", tri]
+    few, full = (cwp.Renderer(cwp.Setup(args + ["--blocks_per_cu", b])) for b in ("1", "0"))
+    s = cwp.Setup(args)
+    rng = np.random.default_rng(n)
+    v = s.array(cwp.ARR_VERTICES)
+    lo, hi = v.min(0), v.max(0)
+    rays = np.empty((n, 8), np.float32)
+    rays[:, 0:3] = rng.uniform(lo - 0.1, hi + 0.1, (n, 3))
+    d = rng.normal(size=(n, 3))
+    d[:n // 2] = np.abs(d[:n // 2])   # like rays first: the waves' first chunks are traced whole
+    rays[:, 4:7] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays[:, 3] = np.where(rng.random(n) < 0.3, rng.uniform(0.0, 0.2, n), 0.0)      # near ends
+    rays[:, 7] = np.where(rng.random(n) < 0.3, rng.uniform(0.2, 1.0, n), 1e30)     # far ends
+    close = few.trace(rays)
+    np.testing.assert_array_equal(close.view(np.uint32), full.trace(rays).view(np.uint32))
+    hit = close[:, 3].view(np.int32) >= 0
+    assert 0.2 < hit.mean() < 0.95
+    np.testing.assert_array_equal(few.trace(rays, any_hit=True)[:, 3].view(np.int32) >= 0, hit)
+    sc, _ = po.scene_from_setup(s)
+    o = sc.trace(rays)
+    same = close[:, 3].view(np.int32) == o[:, 3].view(np.int32)
+    assert same.mean() >= 0.9999
+    both = same & hit
+    assert (np.abs(close[both, 0] - o[both, 0]) <= 1e-5 * np.abs(o[both, 0])).all()
