@@ -27,12 +27,12 @@ LIGHTING = ["--sun_to", "0.608749", "-0.42625", "0.669131", "--sun_rgb", "3", "3
 
 
 def workload_args(width, height, batch, bounces, tri, variant, stack, blocks_per_cu=0, bounce_waves=8, fuse=1,
-                  persistent=0, shadow_refill=0, sort=0, tail=-1, tail_levels=2):
+                  persistent=-1, shadow_refill=-1, sort=0, tail=-1, tail_levels=0):
     return ["--gen", "terrain", "--width", str(width), "--height", str(height), "--batch", str(batch), "--spp", str(batch),
             "--bounces", str(bounces), "--variant", variant, "--tri", tri, "--filter", "box", "--stack", str(stack),
             "--blocks_per_cu", str(blocks_per_cu), "--bounce_waves", str(bounce_waves), "--fuse", str(fuse),
             "--persistent", str(persistent), "--shadow_refill", str(shadow_refill), "--sort", str(sort),
-            "--tail", str(tail), "--tail_levels", str(tail_levels)] + LIGHTING
+            "--tail", str(tail)] + (["--tail_levels", str(tail_levels)] if tail_levels else []) + LIGHTING
 
 
 def algorithmic_bytes(st, npaths, sort=0):
@@ -354,7 +354,7 @@ def bench_jobs(args):
     print("bench: %d scenes (%s tris) set up in %.1f s" % (len(setups), ",".join(str(t) for t in tris),
                                                          time.perf_counter() - t0), file=sys.stderr, flush=True)
     jobs = job_stream(args.jobs, len(setups), args.job_seed, args.job_res, args.job_spp)
-    srv = cwp.Server(variant=8, bounces=6, full=int(args.full), tail_lanes=args.tail, tail_levels=args.tail_levels)
+    srv = cwp.Server(variant=8, bounces=6, full=int(args.full), tail_lanes=args.tail, tail_levels=args.tail_levels or 2)
     for s in setups:
         srv.add_scene(s)
     warm_up(srv, jobs)
@@ -398,7 +398,7 @@ def bench_serve(args):
     import cwp
     setups = make_setups(job_stream_scenes(args.job_scenes, args.job_seed, full=bool(args.full)))
     jobs = job_stream(args.jobs, len(setups), args.job_seed, args.job_res, args.job_spp)
-    srv = cwp.Server(variant=8, bounces=6, full=int(args.full), tail_lanes=args.tail, tail_levels=args.tail_levels)
+    srv = cwp.Server(variant=8, bounces=6, full=int(args.full), tail_lanes=args.tail, tail_levels=args.tail_levels or 2)
     for s in setups:
         srv.add_scene(s)
     warm_up(srv, jobs)
@@ -440,16 +440,17 @@ def main():
     ap.add_argument("--bounce-waves", type=int, default=8)
     ap.add_argument("--blocks-per-cu", type=int, default=0)
     ap.add_argument("--fuse", type=int, default=1, help="1: fused trace+shade kernel; 0: split trace and shade kernels")
-    ap.add_argument("--persistent", type=int, default=0, help="lanes refilled with new rays mid-traversal: 1 split "
-                    "trace / shade kernels, 2 the fused kernel")
-    ap.add_argument("--shadow-refill", type=int, default=0, help="1: shadow kernel refills idle lanes mid-traversal")
+    ap.add_argument("--persistent", type=int, default=-1, help="lanes refilled with new rays mid-traversal: 0 no, 1 split "
+                    "trace / shade kernels, 2 the fused kernel, -1 the library's automatic setting")
+    ap.add_argument("--shadow-refill", type=int, default=-1, help="1: shadow kernel refills idle lanes mid-traversal, 0: a "
+                    "ray per lane, -1 automatic")
     ap.add_argument("--sort", type=int, default=2, help="continuation order: 0 as appended; 1 every bounce's grouped by "
                     "direction bucket per partition; 2 the first bounce's grouped by elevation within each pixel")
     ap.add_argument("--tail", type=int, default=-1, help="straggler hand-off: a trace+shade or shadow wave hands its "
                     "tracing lanes to a tail kernel once fewer than this many remain (0 off, -1 the library's automatic "
                     "setting); the frame workloads, the job stream and serving")
-    ap.add_argument("--tail-levels", type=int, default=2, help="hand-off levels: 1, or 2 (the tail kernels hand their "
-                    "own stragglers on)")
+    ap.add_argument("--tail-levels", type=int, default=0, help="hand-off levels: 1, or 2 (the tail kernels hand their "
+                    "own stragglers on); 0: frames 2 with an explicit --tail, 1 with the automatic one, servers 2")
     ap.add_argument("--cpu-spp", type=int, default=40)
     ap.add_argument("--workload", default="terrain", choices=["terrain", "instances", "jobs", "serve", "hploc"],
                     help="terrain: the diffuse frame (headline), followed by the mixed job stream unless --no-jobs; "
@@ -511,9 +512,9 @@ def main():
             out["serve"], out["tail_lanes"] = bench_serve(args)
         print(json.dumps(out), flush=True)
         return
-    if args.sort == 2 and (args.fuse == 0 or args.persistent):
+    if args.sort == 2 and (args.fuse == 0 or args.persistent > 0):
         args.sort = 0   # the first-bounce sort runs with the fused kernel only
-    if args.tail > 0 and (args.fuse == 0 or args.persistent or args.variant != "bvh8"):
+    if args.tail > 0 and (args.fuse == 0 or args.persistent > 0 or args.variant != "bvh8"):
         args.tail = 0   # the hand-off resumes BVH8 traversals of the fused kernel only
     print("bench: setting up scene", file=sys.stderr, flush=True)
     s = cwp.Setup(workload_args(args.width, args.height, args.batch, args.bounces, args.tri, args.variant, args.stack,
@@ -543,6 +544,8 @@ def main():
     bytes_bounce = sum(algorithmic_bytes(f, npaths, args.sort) for f in frames)
     achieved = bytes_bounce / (bounce_ms * 1e-3) / 1e9
     last = frames[-1]
+    ran = r.frame_json(last)   # the schedule that ran
+    fused = args.fuse and not ran["persistent"]
     out = {
         "metric": "Grays/s on 720p 117k-tri diffuse frame; p50/p99 job latency, batched vs plain",
         "value": round(grays, 4),
@@ -562,8 +565,8 @@ def main():
                    "width": args.width, "height": args.height, "spp": args.batch, "batch": args.batch,
                    "bounces": args.bounces, "bvh": args.variant, "tri": args.tri, "filter": "box",
                    "stack_lds": args.stack, "bounce_waves": args.bounce_waves, "bvh_nodes": info["num_nodes"],
-                   "kernels": {1: "persistent-split", 2: "persistent-fused"}.get(args.persistent, "fused" if args.fuse else "split"),
-                   "shadow_refill": args.shadow_refill, "sort": args.sort, "tail": r.frame_json(last)["tail"]},
+                   "kernels": {1: "persistent-split", 2: "persistent-fused"}.get(ran["persistent"], "fused" if args.fuse else "split"),
+                   "shadow_refill": args.shadow_refill, "sort": args.sort, "tail": ran["tail"]},
         "rays_per_frame": last["rays_closest"] + last["rays_shadow"],
         "rays_closest": last["rays_closest"], "rays_shadow": last["rays_shadow"],
         "t_bounce_ms": round(last["t_bounce_ms"], 3), "t_shade_ms": round(last["t_shade_ms"], 3),
@@ -571,15 +574,15 @@ def main():
         "t_tail_ms": round(last["t_tail_ms"], 3),
         "roofline": {"bound": "hbm", "kernel": ("trace+shade step per depth: k_bounce_first (depth 0, first-bounce sort fused), "
                                                 "k_bounce with straggler hand-off + k_bounce_tail (depths 1-9)")
-                     if args.fuse and not args.persistent and args.sort == 2 and r.frame_json(last)["tail"] > 0
-                     else "k_bounce (fused camera-ray / trace / shade)" if args.fuse and not args.persistent
-                     else ("k_bounce_refill (fused, refilled lanes)" if args.persistent == 2 else "k_trace_paths + k_shade (split trace / shade)"),
+                     if fused and args.sort == 2 and ran["tail"] > 0
+                     else "k_bounce (fused camera-ray / trace / shade)" if fused
+                     else ("k_bounce_refill (fused, refilled lanes)" if ran["persistent"] == 2 else "k_trace_paths + k_shade (split trace / shade)"),
                      "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 5),
-                     "traffic": measured_traffic("k_bounce") if args.fuse and not args.persistent else None,
+                     "traffic": measured_traffic("k_bounce") if fused else None,
                      "traffic_source": "profiles/k_bounce_terrain720p_traffic.md (rocprofv3 FETCH_SIZE / 0.5 + WRITE_SIZE / 1.0)",
                      "bytes_per_frame": bytes_bounce / args.steps,
-                     "utilisation": measured_utilisation("k_bounce family") if args.fuse and not args.persistent
+                     "utilisation": measured_utilisation("k_bounce family") if fused
                      and args.variant == "bvh8" else None,
                      "avg_launch_ms": round(bounce_ms / max(1, launches), 4)},
         "latency": None,

@@ -410,7 +410,7 @@ int cwp_create_scene(const cwp_scene_desc* d, const cwp_params* p, const cwp_opt
     if (O.sort < 0 || O.sort > 2) return fail(CWP_ERR_ARG, "sort must be 0, 1 or 2");
     if (O.batch < 1) return fail(CWP_ERR_ARG, "batch must be >= 1");
     if (O.fuse != 0 && O.fuse != 1) return fail(CWP_ERR_ARG, "fuse must be 0 or 1");
-    if (O.persistent && O.fuse) return fail(CWP_ERR_ARG, "persistent needs fuse 0");
+    if (O.persistent > 0 && O.fuse) return fail(CWP_ERR_ARG, "persistent needs fuse 0");
     cwp_ctx* c = new (std::nothrow) cwp_ctx();
     if (!c) return fail(CWP_ERR_ARG, "out of host memory");
     if (!c->R.init(S, F, O, err)) { delete c; return fail(CWP_ERR_DEVICE, err); }

@@ -988,7 +988,7 @@ __global__ void __launch_bounds__(kBlock, 8) k_trace_paths(DevScene S, DevPaths 
 // results, and take new rays from the partition's queue, while the other lanes keep their traversal state. A wave
 // therefore does not idle until its longest ray is done, and shading still runs on many lanes at once. Each path's
 // arithmetic is the one of k_bounce (same image); only the order of the appends differs.
-// The default for BVH2 (legacy): its rays need many short node visits, whose counts differ most between a wave's lanes,
+// The automatic choice for BVH2 (legacy): its rays need many short node visits, whose counts differ most between a wave's lanes,
 // and its small node step leaves registers for the state that lives through the shading (6 waves per SIMD; 8 spill more,
 // 4 hide less). 720p terrain, 64 samples, 6 bounces: trace+shade 63.1 -> 44.5 ms, with the refilled shadow kernel (18.6 ->
 // 16.9) 81.9 -> 61.5 per frame. BVH4 (47.6 -> 51.3) and BVH8 (6.4 -> 8.7 at 16 samples) are slower with it.
@@ -1876,6 +1876,7 @@ struct Kernels {
     BounceFn bounceFull = nullptr, bounceFullInst = nullptr;
     // fused trace + shade with persistent lanes (legacy and full integrator)
     BounceFn bounceRefill = nullptr, bounceRefillFull = nullptr;
+    BounceFn bounceRefillAuto = nullptr;   // BVH2: the register budget of the automatic schedule
     JobsFn bounceJobsFull = nullptr;
     // rolling batches
     RollFn bounceRoll = nullptr, bounceRollFull = nullptr, shadowRoll = nullptr;
@@ -1919,7 +1920,8 @@ void pickSL(int waves, Kernels& k) {
     k.shadowJobs = k_shadow_jobs<V, TRI, SL>;
     k.bounceFull = k_bounce<V, TRI, SL, kFullWaves, kOneLevel, true>;
     k.bounceFullInst = k_bounce<V, TRI, SL, kFullWaves, kTlas2, true>;
-    k.bounceRefill = waves >= 8 && V != 2 ? k_bounce_refill<V, TRI, SL, 8, false, kShadeBatch>
+    if constexpr (V == 2) k.bounceRefillAuto = k_bounce_refill<V, TRI, SL, 6, false, kShadeBatch>;
+    k.bounceRefill = waves >= 8 ? k_bounce_refill<V, TRI, SL, 8, false, kShadeBatch>
                                 : (waves >= 6 ? k_bounce_refill<V, TRI, SL, 6, false, kShadeBatch> : k_bounce_refill<V, TRI, SL, 4, false, kShadeBatch>);
     k.bounceRefillFull = k_bounce_refill<V, TRI, SL, kFullWaves, true, kShadeBatch>;
     k.bounceJobsFull = k_bounce_jobs<V, TRI, SL, kFullWaves, true>;

@@ -22,7 +22,7 @@ enum LightMode { kLightMIS = 0, kLightNEE = 1, kLightBSDF = 2 };
 
 constexpr int kTailDefault = 12;   // hand-off threshold in lanes of the automatic setting (measured best of 6-16)
 // Most paths in flight for which a frame runs whole paths in one launch (k_path) instead of a queue per depth, where no
-// hand-off, sort, refill or register budget is asked for. Measured at 1280x720, 6 bounces, queues against k_path, ms per
+// hand-off, sort, refill (or none) or register budget is asked for. Measured at 1280x720, 6 bounces, queues against k_path, ms per
 // frame (1.84 M paths and so on for 2, 3, 4, 6 samples): BVH8 terrain 1.91 / 1.76, 2.37 / 2.37, 2.85 / 3.00, 3.72 / 4.16;
 // boxes 1.88 / 1.90; full integrator 1 sample 1.97 / 1.80, 2 samples 2.85 / 3.01. BVH2 4: 7.44 / 7.04, 6: 9.89 / 9.97, full
 // 2: 6.78 / 6.52, 3: 8.86 / 9.06. BVH4 4: 5.49 / 4.96, 6: 7.30 / 7.04. Two levels 4: 15.5 / 14.8, 6: 20.4 / 20.6, full 3:
@@ -45,17 +45,19 @@ struct RenderOptions {
     int bounceWaves = 8;    // trace+shade kernel: register budget for at least this many waves per SIMD (1, 6 or 8)
     int timeKernels = 1;    // per-launch device-clock timing of the trace/shadow kernels
     int fuse = 1;           // 1: trace and shade in one kernel; 0: a closest-hit trace kernel, then a shade kernel
-    int persistent = 0;     // 1: split kernels whose waves refill idle lanes with new rays mid-traversal (implies fuse 0)
-    int shadowRefill = 0;   // shadow kernel: 1 = refill idle lanes mid-traversal, 0 = one ray per lane per round
+    int persistent = -1;    // idle lanes refilled with new rays mid-traversal: 0 no, 1 split kernels (needs fuse 0), 2 the
+                            // fused trace+shade kernel; -1 automatic (Renderer::init)
+    int shadowRefill = -1;  // shadow kernel: 1 = refill idle lanes mid-traversal, 0 = one ray per lane per round, -1 automatic
     int graph = 0;          // 1: a frame is captured once into a HIP graph and replayed (per-kernel timing off)
     int sort = 0;           // 1: between bounces, group each partition's continuations by direction bucket
     int mortonBits = 0;     // two-level scenes: Morton keys of the per-frame TLAS build (0 adaptive, 30: 10 bits per axis)
     int tlasWidth = 8;      // two-level scenes with BVH8 BLASes: the per-frame TLAS as a BVH2 (2) or a compressed BVH8 (8)
-    int tailLevels = 2;     // hand-off levels: 1 (the tail kernels finish every handed-off traversal) or 2 (they hand
-                            // their own stragglers on to a second tail kernel)
+    int tailLevels = 0;     // hand-off levels: 1 (the tail kernels finish every handed-off traversal) or 2 (they hand
+                            // their own stragglers on to a second tail kernel); 0: 2 with an explicit threshold, 1 with the
+                            // automatic one
     int tail = -1;          // straggler hand-off (BVH8, fused kernel): a trace+shade or shadow wave hands
                             // its tracing lanes to a tail kernel once fewer than this many remain (0: off; 2..64;
-                            // -1: kTailDefault lanes and one level where supported and worth it (kTailMin), else off)
+                            // -1: kTailDefault lanes where supported and worth it (kTailMin), else off)
 };
 
 struct FrameStats {

@@ -277,13 +277,24 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     if (!makeDevLights(S, up, I.S.Lt, err)) return false;
 
     if (O.fuse != 0 && O.fuse != 1) { err = "fuse must be 0 or 1"; return false; }
-    if (O.persistent < 0 || O.persistent > 2) { err = "persistent must be 0, 1 (split kernels) or 2 (fused)"; return false; }
+    if (O.persistent < -1 || O.persistent > 2) { err = "persistent must be -1 (auto), 0, 1 (split kernels) or 2 (fused)"; return false; }
     if (O.persistent == 1 && O.fuse) { err = "persistent traversal 1 runs the split kernels (fuse 0)"; return false; }
     if (O.persistent == 2 && !O.fuse) { err = "persistent traversal 2 runs the fused kernel (fuse 1)"; return false; }
     if (S.variant == 2) pickKernels<2>(O.tri, I.sl, O.bounceWaves, I.kn);
     else if (S.variant == 4) pickKernels<4>(O.tri, I.sl, O.bounceWaves, I.kn);
     else pickKernels<8>(O.tri, I.sl, O.bounceWaves, I.kn);
     I.inst = S.inst != 0;
+    // The automatic schedule, where none is asked for: whole paths in one launch for frames with few paths in flight; else
+    // BVH2 queues refill their lanes (k_bounce_refill's comment; the full integrator's trace+shade kernel has no registers left
+    // for that, 25.6 -> 30.4 ms at 16 samples, its shadow rays do, 10.5 -> 6.9), the others trace one ray per lane.
+    const long long inFlight = (long long)F.cam.w * F.cam.h * std::max(O.batch, 1);
+    const bool automatic = O.persistent == -1 && O.fuse && !O.sort && O.bounceWaves == 8;
+    const bool wholePaths = automatic && O.shadowRefill == -1 && O.tail <= 0 &&
+                            (!I.inst || (O.variant == 8 && O.tlasWidth == 8)) && inFlight <= kPathMax(S.variant, I.inst, S.full != 0);
+    const bool refill = automatic && !wholePaths && S.variant == 2 && !I.inst;
+    const int persistent = O.persistent != -1 ? O.persistent : refill && !S.full ? 2 : 0;
+    const bool shadowRefill = O.shadowRefill != -1 ? O.shadowRefill != 0 : refill;
+    I.O.persistent = persistent; I.O.shadowRefill = shadowRefill;
     if (S.full && (!O.fuse || O.persistent == 1)) {
         err = "the full integrator runs the fused kernel (fuse 1, persistent 0 or 2)"; return false;
     }
@@ -293,11 +304,11 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     I.hostMats = S.mats;
     I.nAlbedo = (int)S.albedo.size();
     if (S.full && !I.inst) {
-        I.bounce = O.persistent == 2 ? I.kn.bounceRefillFull : I.kn.bounceFull; I.shade = nullptr;
-        I.shadow = O.shadowRefill ? I.kn.shadowRefill : I.kn.shadow;
+        I.bounce = persistent == 2 ? I.kn.bounceRefillFull : I.kn.bounceFull; I.shade = nullptr;
+        I.shadow = shadowRefill ? I.kn.shadowRefill : I.kn.shadow;
     } else if (I.inst) {
         // two-level scenes run the fused bounce kernel and the one-ray-per-lane shadow kernel
-        if (!O.fuse || O.persistent) { err = "two-level scenes need the fused kernel (fuse 1, persistent 0)"; return false; }
+        if (!O.fuse || persistent) { err = "two-level scenes need the fused kernel (fuse 1, persistent 0)"; return false; }
         I.meshRoot = S.meshRoot; I.nMesh = (int)S.meshRoot.size();
         Vec4* mb;
         if (!I.upload(mb, S.meshBox, err)) return false;
@@ -317,27 +328,19 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         HIPCHK(hipHostMalloc((void**)&I.hostDepth, 2 * sizeof(int), hipHostMallocDefault));   // TLAS depth, build status
         if (!I.alloc(I.dDepth, 1, err)) return false;
     } else {
-        I.bounce = O.fuse ? (O.persistent == 2 ? I.kn.bounceRefill : I.kn.bounce) : (O.persistent ? I.kn.tracePaths : I.kn.tracePlain);
+        I.bounce = !O.fuse ? (persistent ? I.kn.tracePaths : I.kn.tracePlain)
+                   : persistent != 2 ? I.kn.bounce : O.persistent == -1 ? I.kn.bounceRefillAuto : I.kn.bounceRefill;
         I.shade = O.fuse ? nullptr : k_shade;
-        I.shadow = (O.persistent == 1 || O.shadowRefill) ? I.kn.shadowRefill : I.kn.shadow;
+        I.shadow = (persistent == 1 || shadowRefill) ? I.kn.shadowRefill : I.kn.shadow;
     }
     if (O.tail < -1 || O.tail == 1 || O.tail > kWave) { err = "tail must be -1 (auto), 0 (off) or 2..64 lanes"; return false; }
-    if (O.tailLevels != 1 && O.tailLevels != 2) { err = "tail levels must be 1 or 2"; return false; }
-    const long long inFlight = (long long)F.cam.w * F.cam.h * std::max(O.batch, 1);
-    if (O.tail <= 0 && !O.sort && O.fuse && !O.persistent && !O.shadowRefill && O.bounceWaves == 8 &&
-        (!I.inst || I.tlasWide) && inFlight <= kPathMax(S.variant, I.inst, S.full != 0))
-        I.path = I.inst ? (S.full ? I.kn.pathFullInst8 : I.kn.pathInst8) : (S.full ? I.kn.pathFull : I.kn.path);
-    // BVH2 queues with the default schedule refill their lanes (k_bounce_refill's comment); the full integrator's trace+shade
-    // kernel has no registers left for that (25.6 -> 30.4 ms at 16 samples), its shadow rays do (10.5 -> 6.9)
-    if (S.variant == 2 && !I.inst && O.fuse && !O.persistent && !O.sort && O.bounceWaves == 8) {
-        if (!S.full) I.bounce = I.kn.bounceRefill;
-        I.shadow = I.kn.shadowRefill;
-    }
+    if (O.tailLevels < 0 || O.tailLevels > 2) { err = "tail levels must be 1 or 2 (0: automatic)"; return false; }
+    if (wholePaths) I.path = I.inst ? (S.full ? I.kn.pathFullInst8 : I.kn.pathInst8) : (S.full ? I.kn.pathFull : I.kn.path);
     // two-level scenes hand off between node steps of either level, which needs the BVH8 TLAS
-    const bool tailable = S.variant == 8 && (!I.inst || I.tlasWide) && O.fuse && !O.persistent;
-    // automatic: single-level scenes with many paths in flight, one level
+    const bool tailable = S.variant == 8 && (!I.inst || I.tlasWide) && O.fuse && !persistent;
+    // automatic: single-level scenes with many paths in flight
     I.O.tail = O.tail == -1 ? (tailable && !I.inst && inFlight >= kTailMin ? kTailDefault : 0) : O.tail;
-    const bool second = O.tail != -1 && O.tailLevels == 2;
+    const bool second = O.tailLevels ? O.tailLevels == 2 : O.tail != -1;
     if (I.O.tail) {
         if (!tailable) {
             err = "the straggler hand-off (tail) needs a BVH8 scene (two-level: with the BVH8 TLAS) and the fused kernel "
@@ -355,7 +358,7 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         } else {
             I.bounce = S.full ? I.kn.bounceHandFull : I.kn.bounceHand;
             I.bounceTail = S.full ? I.kn.bounceTailFull : I.kn.bounceTail;
-            if (!O.shadowRefill) { I.shadow = I.kn.shadowHand; I.shadowTail = I.kn.shadowTail; }
+            if (!shadowRefill) { I.shadow = I.kn.shadowHand; I.shadowTail = I.kn.shadowTail; }
             if (second) {
                 I.bounceTail2 = S.full ? I.kn.bounceTail2Full : I.kn.bounceTail2;
                 if (I.shadowTail) I.shadowTail2 = I.kn.shadowTail2;
@@ -373,7 +376,7 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
     I.gridShadow = gridOf((const void*)I.shadow);
     I.gridTrace = std::max(gridOf((const void*)I.kn.trace[0]), gridOf((const void*)I.kn.trace[1]));
     I.gridTraceMany = std::max(gridOf((const void*)I.kn.traceMany[0]), gridOf((const void*)I.kn.traceMany[1]));
-    if (O.sort == 2 && !I.inst && O.fuse && !O.persistent) {
+    if (O.sort == 2 && !I.inst && O.fuse && !persistent) {
         I.bounceFirst = S.full ? I.kn.bounceFirstFull : I.kn.bounceFirst;
         int b = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, (const void*)I.bounceFirst, kFirstTile, 0) != hipSuccess || b < 1) b = 1;
@@ -420,7 +423,7 @@ bool Renderer::init(const SceneUpload& S, const FrameParams& F, const RenderOpti
         return false;
     if (!O.fuse && !I.alloc(I.P.H, NK, err)) return false;
     if (O.sort < 0 || O.sort > 2) { err = "sort must be 0, 1 or 2"; return false; }
-    if (O.sort == 2 && (!O.fuse || O.persistent)) { err = "sort 2 (first-bounce sort) needs the fused kernel (fuse 1, persistent 0)"; return false; }
+    if (O.sort == 2 && (!O.fuse || persistent)) { err = "sort 2 (first-bounce sort) needs the fused kernel (fuse 1, persistent 0)"; return false; }
     if (O.sort) {
         if (!I.alloc(I.P.stO, NK, err) || !I.alloc(I.P.stD, NK, err) || !I.alloc(I.P.stT, NK, err) ||
             !I.alloc(I.P.qk, NK, err)) return false;

@@ -108,7 +108,10 @@ bool parseArgs(int argc, const char* const* argv, Args& A, std::string& err) {
         else if (k == "--env_out") ok = str(A.envOut);
         else if (k == "--sort") ok = inum(A.sort);
         else if (k == "--tail") ok = inum(A.tail);
-        else if (k == "--tail_levels") ok = inum(A.tailLevels);
+        else if (k == "--tail_levels") {
+            ok = inum(A.tailLevels);
+            if (ok && A.tailLevels != 1 && A.tailLevels != 2) { err = "--tail_levels must be 1 or 2"; return false; }
+        }
         else if (k == "--devloop") {
             int v = 0; ok = inum(v);
             if (ok && v) { err = k + " selects an experimental variant of the reference that this renderer does not provide"; return false; }
@@ -139,13 +142,12 @@ bool parseArgs(int argc, const char* const* argv, Args& A, std::string& err) {
     if (A.genTextures < 0 || A.genTextures > 8192) { err = "--gen_textures must be 0 (off) or an image size up to 8192"; return false; }
     if (A.collapse != "sah") { err = "--collapse must be sah"; return false; }
     if (A.fuse < -1 || A.fuse > 1) { err = "--fuse must be 0 (split trace and shade kernels) or 1 (fused)"; return false; }
-    if (A.persistent < 0 || A.persistent > 2) {
-        err = "--persistent must be 0, 1 (split kernels with refilled lanes) or 2 (fused kernel with refilled lanes)"; return false;
+    if (A.persistent < -1 || A.persistent > 2) {
+        err = "--persistent must be -1 (auto), 0, 1 (split kernels with refilled lanes) or 2 (fused kernel with refilled lanes)"; return false;
     }
-    if (A.shadowRefill != 0 && A.shadowRefill != 1) { err = "--shadow_refill must be 0 or 1"; return false; }
+    if (A.shadowRefill < -1 || A.shadowRefill > 1) { err = "--shadow_refill must be -1 (auto), 0 or 1"; return false; }
     if (A.sort < 0 || A.sort > 2) { err = "--sort must be 0, 1 or 2"; return false; }
     if (A.tail < -1 || A.tail == 1 || A.tail > 64) { err = "--tail must be -1 (auto), 0 (off) or 2..64 lanes"; return false; }
-    if (A.tailLevels != 1 && A.tailLevels != 2) { err = "--tail_levels must be 1 or 2"; return false; }
     if (A.fuse < 0) A.fuse = 1;
     if (A.persistent == 1) A.fuse = 0;   // persistent traversal 1 runs in the split trace kernel
     if (A.persistent == 2) A.fuse = 1;   // 2: the fused trace+shade kernel with refilled lanes
@@ -657,7 +659,7 @@ std::string frameJson(const SceneSetup& Z, const Renderer& R, const FrameStats& 
              "\"instances\":%d,\"flatten\":%d,\"frame\":%d,\"tlas_ms\":%.3f,\"tlas\":\"%s\",\"bins\":%d,\"stack_lds\":%d,"
              "\"t_bounce_ms\":%.3f,\"t_shade_ms\":%.3f,\"t_shadow_ms\":%.3f,\"rays_hit\":%.0f,\"rays_miss\":%.0f,\"rays_cont\":%.0f,\"shadow_unoccluded\":%.0f,"
              "\"bvh_cache\":\"%s\",\"t_sort_ms\":%.3f,\"tail\":%d}",
-             rep, Z.variant, A.tri.c_str(), A.persistent, A.sort, A.fuse, Z.reportLeaf, A.batch, Z.sceneName.c_str(), Z.M.f.size(), Z.nNodes,
+             rep, Z.variant, A.tri.c_str(), R.options().persistent, A.sort, A.fuse, Z.reportLeaf, A.batch, Z.sceneName.c_str(), Z.M.f.size(), Z.nNodes,
              Z.nodeBytes, Z.maxDepth, Z.bvhS, A.w, A.h, A.spp, A.bounces, st.rays, st.shadowRays, tot, st.traceMs, st.frameMs,
              st.traceMs > 0 ? tot / (st.traceMs * 1e3) : 0.0, st.frameMs > 0 ? tot / (st.frameMs * 1e3) : 0.0,
              st.rays / ((double)N * A.spp), R.vramMB, R.gridBlocks, R.gpuName.c_str(), A.filterBH ? "blackman-harris1.5" : "box",

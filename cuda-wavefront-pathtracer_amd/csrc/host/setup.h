@@ -23,11 +23,11 @@ struct Args {
     std::string integrator = "auto", builder = "sah", collapse = "sah";
     int genBoxes = -1, genGrid = 242; uint64_t genSeed = 1;
     int fuse = -1, leaf = 4, bins = 16, batch = 64, synthetic = 0, frame = 0, w = 512, h = 512, spp = 256, bounces = 8;
-    int persistent = 0, shadowRefill = 0, filterBH = 1, smooth = 1, warm = 8, reps = 1, stack = 8, blocksPerCU = 0, timeKernels = 1;
+    int persistent = -1, shadowRefill = -1, filterBH = 1, smooth = 1, warm = 8, reps = 1, stack = 8, blocksPerCU = 0, timeKernels = 1;
     int bounceWaves = 8;
     int sort = 0;                    // continuations grouped by direction bucket between bounces (same image)
     int tail = -1;                   // straggler hand-off threshold in lanes (-1 auto, 0 off; same image)
-    int tailLevels = 2;              // hand-off levels (1 or 2)
+    int tailLevels = 0;              // hand-off levels (1 or 2; 0: 2 with an explicit threshold, 1 with the automatic one)
     // full material integrator (reference: scene_setup.h:20-22)
     std::string materials, env, lightSampling = "mis", envSampling = "importance";
     float envStrength = -1.f, envRot = -1e30f;   // unset: the lighting file's (or 1, 0)

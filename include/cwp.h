@@ -55,7 +55,9 @@ typedef struct cwp_params {
 typedef struct cwp_frame_stats {
     double rays_closest, rays_shadow;  /* rays traced: camera + continuation, shadow */
     double t_trace_ms, t_frame_ms;     /* trace+shadow kernel time, whole frame (hipEvent pair) */
-    double t_bounce_ms, t_shadow_ms;   /* fused trace+shade kernels, shadow kernels */
+    double t_bounce_ms, t_shadow_ms;   /* fused trace+shade kernels, shadow kernels. Frames with few paths in flight run
+                                          whole paths in one launch per pass (cwp_options.persistent -1): its time,
+                                          shadow rays included, is t_bounce_ms, and t_shadow_ms and shadow_launches are 0 */
     int bounce_launches, shadow_launches;
     double rays_hit, rays_miss, rays_cont, shadow_unoccluded;
     double camera_miss;               /* camera rays that miss (rays_miss includes them) */
@@ -118,11 +120,18 @@ typedef struct cwp_options {
     int batch;           /* samples per pixel in flight per wavefront pass */
     int bounces;         /* maximum bounce depth (camera hit = depth 0), 0..64 */
     int fuse;            /* 1: trace and shade in one kernel; 0: split trace and shade kernels */
-    int persistent;      /* waves refill idle lanes with new rays: 1 split kernels (needs fuse 0), 2 fused kernel */
-    int shadow_refill;   /* 1: the shadow kernel refills idle lanes mid-traversal */
+    int persistent;      /* waves refill idle lanes with new rays: 0 no, 1 split kernels (needs fuse 0), 2 fused kernel;
+                            -1 (default) automatic, where neither fuse 0, sort nor another register budget is asked for:
+                            frames with few paths in flight (1-4 million by layout and integrator; no hand-off, shadow_refill
+                            -1) run whole paths in one launch, whose idle lanes take new paths; larger single-level BVH2
+                            frames refill (the full integrator's shadow rays only); others do not. Same images. */
+    int shadow_refill;   /* 1: the shadow kernel refills idle lanes mid-traversal, 0: one ray per lane, -1 (default)
+                            automatic: as persistent -1 says, else 0 */
     int stack_lds;       /* LDS traversal-stack entries per lane: 8, 16 or 32 (deeper entries spill to HBM) */
     int blocks_per_cu;   /* workgroups per CU of the persistent grids (0 = occupancy limit) */
-    int bounce_waves;    /* fused kernel register budget: at least this many waves per SIMD (1, 6 or 8) */
+    int bounce_waves;    /* register budget of the single-level legacy fused kernel: at least this many waves per SIMD (1, 6
+                            or 8). The full integrator's and two-level scenes' kernels have their own (6), and so have,
+                            with 8, the kernels of persistent -1 (whole paths 5 or 4, the refilled BVH2 kernel 6) */
     int time_kernels;    /* per-launch device-clock timing (t_bounce_ms, t_shade_ms, t_shadow_ms) */
     int graph;           /* 1: each frame replays a captured HIP graph (per-launch timing off) */
     int sort;            /* continuations reordered before they are traced (reference option --sort,
@@ -131,7 +140,9 @@ typedef struct cwp_options {
                             bucket within each pixel's samples (fused kernel only) */
     int tail_lanes;      /* straggler hand-off (compressed BVH8, fused kernel): once fewer than
                             this many lanes of a trace+shade wave are still tracing, their traversals are handed to a
-                            tail kernel that resumes them in full waves (same results); 0 off, 2..64 */
+                            tail kernel that resumes them in full waves, with 2..64 lanes in two levels (same results);
+                            0 off; -1 (default): 12 lanes and one level for single-level frames of at least 2^25 paths
+                            in flight, else off */
 } cwp_options;
 
 /* Scene and BVH summary of a setup. */

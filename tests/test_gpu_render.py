@@ -447,15 +447,44 @@ def test_chunks_handed_out_equal_one_chunk_per_wave(extra):
 @pytest.mark.parametrize("extra", [[], ["--gen_materials", "3", "--gen_env", "64,32,1.5,2"]])
 def test_bvh2_default_schedule_equals_plain_queues(extra):
     """BVH2 frames with more paths than whole-path launches take refill their lanes by default; image and ray counts are
-    those of the plain queue kernels, which a register budget asks for."""
+    those of the plain queue kernels, which a register budget or persistent 0 asks for; an explicit schedule is the one
+    that runs (the JSON's persistent; the refilling kernel of a budget of 8 waves has the plain one's grid)."""
     print("case", extra, flush=True)
     args = ["--gen", "boxes", "--gen_boxes", "60", "--width", "1001", "--height", "701", "--batch", "6", "--bounces", "3",
             "--variant", "bvh2"] + extra
-    a, b = (cwp.Renderer(cwp.Setup(args + o)) for o in ([], ["--bounce_waves", "6"]))
-    x, y = a.render(6), b.render(6)
-    np.testing.assert_array_equal(a.accum(), b.accum())
-    for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
-        assert x[key] == y[key], key
+    full = bool(extra)
+    ran = {}
+    for o in ((), ("--bounce_waves", "6"), ("--persistent", "0"), ("--persistent", "0", "--shadow_refill", "1"),
+              ("--persistent", "2"), ("--shadow_refill", "0")):
+        r = cwp.Renderer(cwp.Setup(args + list(o)))
+        st = r.render(6)
+        ran[o] = (r.accum(), st, r.frame_json(st)["persistent"], r.grid_blocks)
+        r.close()
+    img, st, _, _ = ran["--bounce_waves", "6"]
+    for o, (a, x, _, _) in ran.items():
+        np.testing.assert_array_equal(a, img, err_msg=str(o))
+        for key in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
+            assert x[key] == st[key], (o, key)
+    assert [ran[o][2] for o in ran] == [0 if full else 2, 0, 0, 0, 2, 0 if full else 2]
+    if not full:
+        assert ran["--persistent", "0"][3] == ran["--persistent", "2"][3] > ran[()][3]
+
+
+def test_tail_levels_asked_for_with_the_automatic_hand_off():
+    """The automatic hand-off (from 2^25 paths in flight) has one level; --tail_levels 2 beside it gives two, whose records
+    take memory of their own. Same image."""
+    print("case tail levels", flush=True)
+    args = ["--gen", "boxes", "--gen_boxes", "60", "--width", "1024", "--height", "1024", "--batch", "32", "--bounces", "1"]
+    out = []
+    for o in ([], ["--tail_levels", "1"], ["--tail_levels", "2"]):
+        r = cwp.Renderer(cwp.Setup(args + o))
+        st = r.render(32)
+        out.append((r.vram_mb, r.accum()))
+        assert r.frame_json(st)["tail"] == 12
+        r.close()
+    assert abs(out[0][0] - out[1][0]) < 16 and out[2][0] > out[0][0] + 32
+    for k in (1, 2):
+        np.testing.assert_array_equal(out[k][1], out[0][1])
 
 
 @pytest.mark.parametrize("variant,tri,n", [(8, "woop", 16384), (8, "woop", 16385), (8, "woop", 100003), (8, "watertight", 40001),

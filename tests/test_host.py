@@ -57,7 +57,13 @@ def test_version_and_error_string():
         with pytest.raises(cwp.CwpError, match="--tail"):
             cwp.Setup(["--gen", "boxes", "--tail", bad])
     cwp.Setup(["--gen", "boxes", "--sort", "1", "--devloop", "0", "--morton_bits", "30", "--tlas", "bvh2"])
+    for arg, bads in (("--tail_levels", ("0", "3", "-1")), ("--persistent", ("-2",)), ("--shadow_refill", ("2", "-2"))):
+        for bad in bads:
+            with pytest.raises(cwp.CwpError, match=arg):
+                cwp.Setup(["--gen", "boxes", arg, bad])
+    cwp.Setup(["--gen", "boxes", "--persistent", "-1", "--shadow_refill", "-1", "--tail_levels", "1"])
     assert cwp.Options.default().sort == 0
+    assert (cwp.Options.default().persistent, cwp.Options.default().shadow_refill) == (-1, -1)   # automatic
     assert cwp.Options.default().tail_lanes == -1   # automatic: on where the schedule supports it
 
 
