@@ -177,7 +177,7 @@ def test_overlapping_instances(tri, stack, tail, count):
     assert ((gt == ot) & (gi == oi)).mean() >= 0.999
     assert np.array_equal(r.trace_inst(rays, any_hit=True)[0][:, 3].view(np.int32) >= 0, gt >= 0)
     r.render(4)
-    plain = cwp.Renderer(cwp.Setup(args + ["--tail", "0"]))
+    plain = cwp.Renderer(cwp.Setup(args + ["--tail", "0", "--persistent", "0"]))
     plain.set_instances(inst)
     plain.render(4)
     np.testing.assert_array_equal(r.accum(), plain.accum())
@@ -211,6 +211,42 @@ def test_two_level_queries_of_more_rays_than_lanes(tri, tlas, n):
     np.testing.assert_array_equal(ai >= 0, hit)
     o, oi = oracle_scene(s, 0, {"mt": 0, "woop": 1, "watertight": 2}[tri]).trace_inst(rays)
     assert ((g[:, 3].view(np.int32) == o[:, 3].view(np.int32)) & (gi == oi)).mean() >= 0.999
+
+
+@pytest.mark.parametrize("full", [False, True])
+def test_two_level_queues_equal_whole_paths(full):
+    """The queue kernels of two-level scenes, with one workgroup per CU (the counters hand most chunks out, to other
+    partitions' waves too) and the full grid, against whole paths in one launch: images and ray counts bit for bit, on two
+    frames. A frame of the full integrator with more paths than whole-path launches take uses them by itself."""
+    print("case two-level queues", full, flush=True)
+    extra = ["--gen_materials", "2", "--gen_env", "64,32,1.5,2"] if full else []
+    keys = ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss")
+
+    def frames(args, spp, n=2):
+        r = cwp.Renderer(cwp.Setup(args))
+        out = []
+        for f in range(n):
+            r.set_frame(f)
+            st = r.render(spp, f * spp)
+            out.append((r.accum(), [st[k] for k in keys], st["shadow_launches"]))
+        r.close()
+        return out
+
+    args = ARGS[:-4] + ["--width", "211", "--height", "157", "--batch", "8", "--bounces", "4", "--graph", "0"] + extra
+    whole = frames(args, 8)
+    assert whole[0][2] == 0
+    for o in (["--persistent", "0"], ["--persistent", "0", "--blocks_per_cu", "1"]):
+        for (a, n, launches), (b, m, _) in zip(frames(args + o, 8), whole):
+            assert launches == 6
+            np.testing.assert_array_equal(a, b)
+            assert n == m
+    if full:
+        args = ARGS[:-4] + ["--width", "1001", "--height", "701", "--batch", "3", "--bounces", "2", "--graph", "0"] + extra
+        (a, n, launches), = frames(args, 3, 1)
+        (b, m, _), = frames(args + ["--tail", "12"], 3, 1)
+        assert launches == 4
+        np.testing.assert_array_equal(a, b)
+        assert n == m
 
 
 FULL = ARGS + ["--gen_materials", "2", "--gen_env", "64,32,1.5,2", "--bounces", "3"]

@@ -144,15 +144,16 @@ def test_thin_lens_render_matches_oracle():
 
 @pytest.mark.parametrize("scene,variant", [("terrain", 8), ("boxes", 2), ("boxes", 4)])
 def test_kernel_schedules_give_the_same_image(scene, variant):
-    """Fused trace+shade, split trace/shade, split with persistent refilling lanes, and the shadow kernel with and
-    without refilling compute every path with the same arithmetic in the same order per path: images and counters are
+    """Fused trace+shade, split trace/shade, split and fused with persistent refilling lanes, the shadow kernel with and
+    without refilling, and the automatic schedule (whole paths in one launch for a frame this small) compute every path with the same arithmetic in the same order per path: images and counters are
     bit-identical, and match the oracle."""
     print("case", scene, variant, flush=True)
     spp, batch, bounces = 8, 8, 5
     base = SCENES[scene] + ["--variant", "bvh%d" % variant, "--batch", str(batch), "--bounces", str(bounces),
                             "--spp", str(spp)]
     out = {}
-    schedules = [("fused", ["--fuse", "1", "--shadow_refill", "0"]), ("fused-refill", ["--fuse", "1"]),
+    schedules = [("fused", ["--fuse", "1", "--persistent", "0", "--shadow_refill", "0"]), ("automatic", ["--fuse", "1"]),
+                 ("fused-refill", ["--fuse", "1", "--persistent", "0", "--shadow_refill", "1"]),
                  ("split", ["--fuse", "0", "--shadow_refill", "0"]), ("persistent", ["--persistent", "1"]),
                  ("fused-persistent", ["--persistent", "2"])]
     for name, extra in schedules:
@@ -160,10 +161,10 @@ def test_kernel_schedules_give_the_same_image(scene, variant):
         r = cwp.Renderer(s)
         st = r.render(spp)
         out[name] = (r.accum(), st)
-        assert r.frame_json(st)["fuse"] == (1 if name.startswith("fused") else 0)
+        assert r.frame_json(st)["fuse"] == (0 if name in ("split", "persistent") else 1)
         r.close()
     img0, st0 = out["fused"]
-    for name in ("fused-refill", "split", "persistent", "fused-persistent"):
+    for name in ("automatic", "fused-refill", "split", "persistent", "fused-persistent"):
         img, st = out[name]
         np.testing.assert_array_equal(img, img0, err_msg=name)
         for k in ("rays_closest", "rays_shadow", "rays_miss", "rays_cont", "shadow_unoccluded", "camera_miss"):
@@ -200,7 +201,8 @@ def test_sorted_continuations_give_the_same_image(name, args):
     out = {}
     fused = "--fuse" not in args and "--persistent" not in args
     for sort in (0, 1, 2) if fused else (0, 1):
-        r = cwp.Renderer(cwp.Setup(base + ["--sort", str(sort)]))
+        plain = ["--persistent", "0"] if fused and sort == 0 else []   # the queue kernels, not whole paths in one launch
+        r = cwp.Renderer(cwp.Setup(base + ["--sort", str(sort)] + plain))
         frames = []
         for f in range(2):
             if name == "instances":
@@ -344,7 +346,8 @@ def test_straggler_hand_off_gives_the_same_image(name, args, sorts):
         out = {}
         for tail, levels in ((0, 1), (8, 2), (64, 2), (8, 1), (64, 1)):
             print("case", name, "sort", sort, "tail", tail, "levels", levels, flush=True)
-            r = cwp.Renderer(cwp.Setup(base + ["--sort", str(sort), "--tail", str(tail), "--tail_levels", str(levels)]))
+            r = cwp.Renderer(cwp.Setup(base + ["--sort", str(sort), "--tail", str(tail), "--tail_levels", str(levels),
+                                               "--persistent", "0"]))
             frames = []
             for f in range(2):
                 if name.startswith("instances"):
@@ -429,6 +432,8 @@ def test_whole_paths_equal_the_queue_kernels(scene, variant, tri, size, extra):
                                    ["--variant", "bvh2", "--bounce_waves", "6"], ["--variant", "bvh4", "--bounce_waves", "6"],
                                    ["--variant", "bvh2", "--persistent", "2", "--shadow_refill", "1"],
                                    ["--tail", "0", "--persistent", "2", "--shadow_refill", "1"],
+                                   ["--persistent", "0"], ["--sort", "1"], ["--variant", "bvh2", "--persistent", "0"],
+                                   ["--persistent", "0", "--gen_materials", "3", "--gen_env", "64,32,1.5,2"],
                                    ["--tail", "12", "--gen_materials", "3", "--gen_env", "64,32,1.5,2"]])
 def test_chunks_handed_out_equal_one_chunk_per_wave(extra):
     """With one workgroup per CU most chunks of a launch are handed out by the partitions' counters, to other partitions'
