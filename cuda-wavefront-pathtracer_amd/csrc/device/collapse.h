@@ -10,9 +10,9 @@
 //  2. the collapse's cost tables bottom-up: one lane per leaf climbs to the root, the second lane to reach a node
 //     computes it from both children (cost of the subtree as 1..7 wide-tree roots, decisions, the split of 8 roots),
 //     with device-coherent hand-over as in the H-PLOC climb;
-//  3. the wide nodes top-down, one launch per level (its range read from device memory; the host checks once per 8
-//     levels): each node's children (the decisions' roots), the greedy octant
-//     slot assignment, leaf / internal flags;
+//  3. the wide nodes top-down, eight lanes per node: the first levels, or all of a small tree's, in one workgroup, the others
+//     a launch each (its range read from device memory), 16 levels and the steps below queued before the host looks at the
+//     counts: each node's children (the decisions' roots), the greedy octant slot assignment, leaf / internal flags;
 //  4. the host's numbering: its job stack visits a node's internal children in decreasing slot order and appends
 //     each node's children (and leaf primitives) when it pops the node, so child bases and triangle bases are prefix
 //     sums over that order, computed from subtree totals (bottom-up) and offsets (top-down);

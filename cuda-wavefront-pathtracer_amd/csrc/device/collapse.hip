@@ -14,9 +14,12 @@ constexpr unsigned char kDecLeaf = 0, kDecNode = 1, kDecPrev = 2, kDecDist = 10;
 constexpr float kInf = 3e38f;
 constexpr int kWaitVmcnt0 = 0x0F70;      // s_waitcnt vmcnt(0)
 
-// The wide levels 0 .. kTopLevels - 1 (at most 8^l nodes each), and every level of a tree of at most kOneBlock primitives,
-// run in one workgroup: a launch per level costs more than such a level's work.
-constexpr int kTopLevels = 4, kOneBlock = 8192;
+// The wide levels 0 .. kTopLevels - 1 (at most 8^l nodes each), and every level of a tree of at most kOneBlock primitives, run
+// in one workgroup: a launch per level, three with the numbering, costs more than such a level's work. Whole collapse of n
+// random boxes, ms: kTopLevels 2 / 4 / 6 at n = 12,000 0.358 / 0.395 / 0.437, 100,000 0.421 / 0.465 / 1.44, 500,000 0.571 / 0.618
+// / 3.84 (level 2 has up to 64 nodes, 8 waves' work, but level 3 up to 512). One workgroup / launches: 1,000 primitives 0.220 /
+// 0.281, 8,192 0.320 / 0.366, 12,000 0.369 / 0.380, 20,000 0.453 / 0.393.
+constexpr int kTopLevels = 2, kOneBlock = 8192;
 
 // scratch arrays carved out of one allocation (binary nodes: N = 2n - 1; wide nodes: at most n)
 struct Scratch {
