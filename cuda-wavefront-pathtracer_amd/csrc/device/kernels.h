@@ -5,8 +5,9 @@
 //
 // Design (MI355X-first, not the reference's launch structure):
 //  * Persistent grids: every kernel launches a fixed grid of single-wave workgroups sized to the occupancy limit and
-//    walks its queue in wave-sized chunks (grid stride). Queue lengths are read from device memory, so a frame is
-//    enqueued once, with no count readback between bounces.
+//    walks its queue in wave-sized chunks: the first is the wave's own, counters hand the others out (Chunks; the split
+//    kernels k_trace_paths and k_shade, and depth 0 with the fused sort, take fixed shares). Queue lengths are read from
+//    device memory, so a frame is enqueued once, with no count readback between bounces.
 //  * Queue compaction per wave: the continuation and shadow decisions are ballots; one lane reserves the wave's block
 //    of slots with a single atomic and every lane writes at its mbcnt rank (reference: per-thread atomicAdd appends,
 //    src/render/wavefront.cu:119,135).
@@ -54,7 +55,8 @@ constexpr int kCTail2 = 8, kCShadowTail2 = 9;
 constexpr int kWPath = 0, kWBounce = 1, kWTail = 2, kWTail2 = 3, kWShadow = 4, kWShadowTail = 5, kWShadowTail2 = 6;
 // Device-clock stamps (64 bits each) in partition 0's line: when the depth's first trace+shade, tail, shade, shadow,
 // shadow-tail and sort launch began (0: no such launch). A launch's time is the next stamp minus its own (k_pass_end).
-// An event record between two launches costs 6-10 us of idle GPU, four of them per depth 0.32 ms of a ten-depth frame.
+// An event record between two launches costs 6-10 us of idle GPU: four of them per depth, six with tail launches, were 0.32 ms
+// of a ten-depth frame.
 constexpr int kCStampBounce = 12, kCStampTail = 14, kCStampShade = 16, kCStampShadow = 18, kCStampShadowTail = 20, kCStampSort = 22;
 
 // Lights and materials of the full integrator (device pointers; null / 0 for the legacy integrator)
@@ -792,10 +794,11 @@ __device__ __forceinline__ ShadeOut shadeSlot(const DevScene& S, const DevPaths&
 }
 
 // One bounce of the legacy integrator over the queue of depth `depth` (depth 0: every path id, camera rays made here),
-// traversal and shading fused. The queue is split into kParts partitions, one per XCD; the waves of XCD x walk
-// partition x, and append their continuations to partition x of the next queue and their shadow rays to partition x of
-// the shadow queue, so a path stays on one XCD (and in its L2) for its whole life. Partition x of the depth-(d+1) queue
-// starts where the depth-d partitions before x end, which bounds it by the rays partition x traced.
+// traversal and shading fused. The queue is split into kParts partitions, one per XCD; the waves of XCD x take partition
+// x's chunks, and the continuations and shadow rays of a chunk go to its own partition of the next queues, so most of a
+// path's life is on one XCD (and in its L2); waves that find no chunk left in their partition help one other (Chunks).
+// Partition x of the depth-(d+1) queue starts where the depth-d partitions before x end, which bounds it by the rays
+// traced from partition x.
 // WAVES: minimum waves per SIMD the register allocation must allow (1 = unconstrained).
 // TAIL (BVH8; two-level scenes with a BVH8 TLAS): straggler hand-off. After each node visit a wave counts its lanes still tracing;
 // once fewer than P.tailLanes are, they stop and write their traversal state as tail records (k_bounce_tail resumes
@@ -995,8 +998,8 @@ __global__ void __launch_bounds__(kBlock, 8) k_trace_paths(DevScene S, DevPaths 
 // arithmetic is the one of k_bounce (same image); only the order of the appends differs.
 // The automatic choice for BVH2 (legacy): its rays need many short node visits, whose counts differ most between a wave's lanes,
 // and its small node step leaves registers for the state that lives through the shading (6 waves per SIMD; 8 spill more,
-// 4 hide less). 720p terrain, 64 samples, 6 bounces: trace+shade 63.1 -> 44.5 ms, with the refilled shadow kernel (18.6 ->
-// 16.9) 81.9 -> 61.5 per frame. BVH4 (47.6 -> 51.3) and BVH8 (6.4 -> 8.7 at 16 samples) are slower with it.
+// 4 hide less). 720p terrain, 16 samples, 6 bounces, one ray per lane / refilled: trace+shade BVH2 16.75 / 12.19 ms, BVH4 12.66 /
+// 16.76, BVH8 6.40 / 9.22; shadow launches (k_shadow_refill) BVH2 4.20 / 3.66, BVH4 2.95 / 4.06, BVH8 1.55 / 1.95.
 template <int V, int TRI, int SL, int WAVES, bool FULL, int REFILL>
 __global__ void __launch_bounds__(kBlock, WAVES) k_bounce_refill(DevScene S, DevPaths P, const FrameParams* __restrict__ Fp,
                                                                  int depth, int smpBase, int K) {

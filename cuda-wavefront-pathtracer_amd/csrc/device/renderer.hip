@@ -3,8 +3,9 @@
 //
 // Design (MI355X-first, not the reference's launch structure):
 //  * Persistent grids: every kernel launches a fixed grid of single-wave workgroups sized to the occupancy limit and
-//    walks its queue in wave-sized chunks (grid stride). Queue lengths are read from device memory, so a frame is
-//    enqueued once, with no count readback between bounces.
+//    walks its queue in wave-sized chunks: the first is the wave's own, counters hand the others out (Chunks; the split
+//    kernels k_trace_paths and k_shade, and depth 0 with the fused sort, take fixed shares). Queue lengths are read from
+//    device memory, so a frame is enqueued once, with no count readback between bounces.
 //  * Queue compaction per wave: the continuation and shadow decisions are ballots; one lane reserves the wave's block
 //    of slots with a single atomic and every lane writes at its mbcnt rank (reference: per-thread atomicAdd appends,
 //    src/render/wavefront.cu:119,135).
@@ -714,7 +715,7 @@ bool Renderer::setInstances(const InstanceRecord* rec, int n, double& tlasMs, st
     int hroot = 0, wideNodes = 0, wideDepth = 0;
     if (!I.tlasB.build(I.dLo, I.dHi, n, I.st, hroot, err, I.O.mortonBits)) return false;
     if (I.tlasWide) {
-        // the collapse checks the H-PLOC tree itself and synchronises with the stream between its levels
+        // the collapse checks the H-PLOC tree itself and synchronises with the stream
         if (!I.tlasC.run(I.tlasB.nodes(), n, I.dTlas80, I.dTlasPrim, I.st, wideNodes, wideDepth, err)) return false;
         k_bvh8_device<<<(wideNodes + 255) / 256, 256, 0, I.st>>>(I.dTlas80, wideNodes, I.dTlas8);
     } else if (!hplocToBVH2(I.tlasB.nodes(), n, I.dTlas, I.st, err)) return false;
