@@ -308,6 +308,27 @@ def test_straggler_hand_off_gives_the_same_images(full, rolling, compact):
             np.testing.assert_array_equal(out[tail][0][k], out[0, 2][0][k], err_msg="tail %s job %d" % (tail, k))
 
 
+@pytest.mark.parametrize("rolling,compact", [(1, 0), (1, 1), (0, 0)])
+def test_hand_off_with_the_watertight_test(rolling, compact):
+    """The hand-off kernels of the watertight triangle test (their ray state is the largest) give the images of no
+    hand-off, with one and two levels."""
+    S = [cwp.Setup(TERRAIN + ["--bounces", "4", "--tri", "watertight"]), cwp.Setup(BOXES + ["--bounces", "4", "--tri", "watertight"])]
+    out = {}
+    for tail, levels in ((0, 2), (12, 1), (64, 2)):
+        print("case watertight hand-off", rolling, compact, tail, levels, flush=True)
+        srv = cwp.Server(variant=8, bounces=4, max_paths=1 << 14, tri_test=2, rolling=rolling, compact=compact, tail_lanes=tail,
+                         tail_levels=levels)
+        for s in S:
+            srv.add_scene(s)
+        imgs, _, st = run_jobs(srv, JOBS, True)
+        out[tail] = (imgs, st["rays"])
+        srv.close()
+    for tail in (12, 64):
+        assert out[tail][1] == out[0][1]
+        for k in range(len(JOBS)):
+            np.testing.assert_array_equal(out[tail][0][k], out[0][0][k], err_msg="tail %d job %d" % (tail, k))
+
+
 def test_live_submissions_from_threads_while_jobs_run():
     """cwp_server_start / cwp_job_submit / cwp_job_poll / cwp_job_result: two threads submit jobs while others are on
     the GPU; every job reaches DONE and its image equals the job rendered alone."""
