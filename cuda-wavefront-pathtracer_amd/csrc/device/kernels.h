@@ -1911,10 +1911,11 @@ struct Kernels {
     RollFn shadowRollHand = nullptr, shadowRollTail = nullptr;
 };
 
-// Waves per SIMD of the rolling steps' legacy hand-off kernels. At 8 (64 registers) the compiler places register spills of
+// Waves per SIMD of the batches' legacy hand-off kernels, which hold job pointers beside the traversal: 6 spill less and are
+// faster than 8 (rolling steps, 24 jobs of 256x256: 9.0 -> 8.0 ms; passes 9.5 -> 7.6). At 8 (64 registers) the compiler places register spills of
 // some of them (watertight test) where a divergent branch has joined but before its lanes are active again: lanes of the
 // other side read stale job pointers and pixels back. At 6 nothing is spilled there (tests/test_kernel_code.py checks it).
-constexpr int kHandRollWaves = 6;
+constexpr int kHandWaves = 6;
 
 template <int V, int TRI, int SL>
 void pickSL(int waves, Kernels& k) {
@@ -1971,22 +1972,22 @@ void pickSL(int waves, Kernels& k) {
         k.shadowHandInst = k_shadow<V, TRI, SL, kTlas8, true>;
         k.shadowTailInst = k_shadow_tail<TRI, SL, 1, kTlas8>;
         k.shadowTail2Inst = k_shadow_tail<TRI, SL, 2, kTlas8>;
-        k.bounceJobsHand = k_bounce_jobs<V, TRI, SL, 8, false, true>;
+        k.bounceJobsHand = k_bounce_jobs<V, TRI, SL, kHandWaves, false, true>;
         k.bounceJobsHandFull = k_bounce_jobs<V, TRI, SL, kFullWaves, true, true>;
-        k.bounceJobsTail = k_bounce_jobs_tail<TRI, SL, 8, false>;
+        k.bounceJobsTail = k_bounce_jobs_tail<TRI, SL, kHandWaves, false>;
         k.bounceJobsTailFull = k_bounce_jobs_tail<TRI, SL, kFullWaves, true>;
         k.shadowJobsHand = k_shadow_jobs<V, TRI, SL, true>;
         k.shadowJobsTail = k_shadow_jobs_tail<TRI, SL, false, DevJobTable>;
-        k.bounceRollHand[0][0] = k_bounce_roll<V, TRI, SL, kHandRollWaves, false, false, true>;
-        k.bounceRollHand[0][1] = k_bounce_roll<V, TRI, SL, kHandRollWaves, false, true, true>;
+        k.bounceRollHand[0][0] = k_bounce_roll<V, TRI, SL, kHandWaves, false, false, true>;
+        k.bounceRollHand[0][1] = k_bounce_roll<V, TRI, SL, kHandWaves, false, true, true>;
         k.bounceRollHand[1][0] = k_bounce_roll<V, TRI, SL, kFullWaves, true, false, true>;
         k.bounceRollHand[1][1] = k_bounce_roll<V, TRI, SL, kFullWaves, true, true, true>;
-        k.bounceRollTail[0][0] = k_bounce_roll_tail<TRI, SL, kHandRollWaves, false, false>;
-        k.bounceRollTail[0][1] = k_bounce_roll_tail<TRI, SL, kHandRollWaves, false, true>;
+        k.bounceRollTail[0][0] = k_bounce_roll_tail<TRI, SL, kHandWaves, false, false>;
+        k.bounceRollTail[0][1] = k_bounce_roll_tail<TRI, SL, kHandWaves, false, true>;
         k.bounceRollTail[1][0] = k_bounce_roll_tail<TRI, SL, kFullWaves, true, false>;
         k.bounceRollTail[1][1] = k_bounce_roll_tail<TRI, SL, kFullWaves, true, true>;
-        k.bounceRollTail2[0][0] = k_bounce_roll_tail<TRI, SL, kHandRollWaves, false, false, 2>;
-        k.bounceRollTail2[0][1] = k_bounce_roll_tail<TRI, SL, kHandRollWaves, false, true, 2>;
+        k.bounceRollTail2[0][0] = k_bounce_roll_tail<TRI, SL, kHandWaves, false, false, 2>;
+        k.bounceRollTail2[0][1] = k_bounce_roll_tail<TRI, SL, kHandWaves, false, true, 2>;
         k.bounceRollTail2[1][0] = k_bounce_roll_tail<TRI, SL, kFullWaves, true, false, 2>;
         k.bounceRollTail2[1][1] = k_bounce_roll_tail<TRI, SL, kFullWaves, true, true, 2>;
         k.shadowRollHand = k_shadow_roll<V, TRI, SL, true>;

@@ -1,4 +1,4 @@
-"""Compiled code of the rolling steps' hand-off kernels (cross-compiled for gfx950, no GPU). Where the two sides of a
+"""Compiled code of the batches' hand-off kernels (cross-compiled for gfx950, no GPU). Where the two sides of a
 divergent branch join, the compiler has been seen to spill registers before the instruction that makes all the lanes
 active again: the lanes of the other side then read stale values back (job pointers, pixels: wrong images or worse). The
 kernels' register budget is chosen so that it does not; this looks for such spills in the assembly."""
@@ -43,15 +43,18 @@ def test_no_spill_before_the_lanes_of_a_join_are_back(tmp_path):
         with open(src, "w") as f:
             f.write('#include "device/kernels.h"\nnamespace cwp { namespace dev {\n')
             for lane in ("false", "true"):
-                f.write("template __global__ void k_bounce_roll<8, %d, 8, kHandRollWaves, false, %s, true>"
+                f.write("template __global__ void k_bounce_roll<8, %d, 8, kHandWaves, false, %s, true>"
                         "(const DevStepTable*, DevPaths, int);\n" % (tri, lane))
                 for level in (1, 2):
-                    f.write("template __global__ void k_bounce_roll_tail<%d, 8, kHandRollWaves, false, %s, %d>"
+                    f.write("template __global__ void k_bounce_roll_tail<%d, 8, kHandWaves, false, %s, %d>"
                             "(const DevStepTable*, DevPaths, int);\n" % (tri, lane, level))
+            f.write("template __global__ void k_bounce_jobs<8, %d, 8, kHandWaves, false, true>(const DevJobTable*, DevPaths, int);\n"
+                    "template __global__ void k_bounce_jobs_tail<%d, 8, kHandWaves, false>(const DevJobTable*, DevPaths, int);\n"
+                    % (tri, tri))
             f.write("}}\n")
         subprocess.run([build.hipcc()] + build.HIP_FLAGS + build.INCLUDES + ["--cuda-device-only", "-S", src, "-o", asm], check=True,
                        stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
-        assert open(asm).read().count("s_endpgm") >= 6
+        assert open(asm).read().count("s_endpgm") >= 8
         return joins_with_early_spills(asm)
 
     with ThreadPoolExecutor(3) as ex:
